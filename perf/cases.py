@@ -25,9 +25,15 @@ from pis_amd import Atoms, Engine, LennardJones, LJGpuManager, Server, workloads
 from pis_amd.box import SimulationBox
 from pis_amd.engine import PinnedArray
 
-# thermostat and barostat of the NVT and NPT runs: chain time constant, and a barostat heavy
-# enough that the box stays near its start over any number of passes
-TAU_T, TAU_P, CHAIN = 0.5, 400.0, 3
+# Thermostat and barostat of the NVT and NPT runs.  The reference's chain sets xi from the
+# kinetic energy's excess over 3 N kB T instead of integrating it, so a step scales the
+# velocities by a power that grows with N / tau^2: a steady run takes tau with sqrt(N).  The
+# barostat is heavy enough that the box stays near its start over any number of passes.
+TAU_P, CHAIN = 400.0, 3
+
+
+def tau_t(n):
+    return max(0.5, 0.03 * math.sqrt(n))
 
 
 def listed():
@@ -159,9 +165,9 @@ def prepare(case, seed):
         eng.compute_potential()
         s["eng"] = eng
         if case.get("ens") == "nvt":
-            eng.nvt_init(case["temp"], case["temp"], TAU_T, CHAIN)
+            eng.nvt_init(case["temp"], case["temp"], tau_t(case["n"]), CHAIN)
         if case.get("ens") == "npt":
-            eng.npt_init(case["temp"], case["temp"], TAU_T, 0.0, TAU_P, CHAIN)
+            eng.npt_init(case["temp"], case["temp"], tau_t(case["n"]), 0.0, TAU_P, CHAIN)
         if case["kind"] == "run":
             s["frame"] = PinnedArray((specs[0].n, 3))
         if mixed:
@@ -378,7 +384,7 @@ class _Exact:
     # from the current forces, not integrated) and its MTK barostat
 
     def chain(self, t0):
-        q = self.kb * t0 * TAU_T * TAU_T
+        q = self.kb * t0 * tau_t(self.n) ** 2
         self.q, self.xi, self.t = [q / 10.0 ** i for i in range(CHAIN)], [0.0] * CHAIN, t0
 
     def chain_half(self, dt):
