@@ -132,14 +132,14 @@ struct SysDev {
     int32_t* cell_count;   // [ncell] atoms per cell while sorting; zero between rebuilds
     int32_t* cell_start;   // [ncell+1], sorted (tile-major) cell ids
     int32_t* nat2sorted;   // [ncell]: natural (cz*ny+cy)*nx+cx -> sorted id
-    int32_t* tile_cell0;   // [ntile+1]
     int32_t* atom_cell;    // [n] sorted cell id of atom (live order) at binning
     int32_t* scat_src;     // [n] scatter slot -> source atom
     uint32_t* scat_key;    // [n] scatter slot -> orig index (sort key, ties)
     double* scat_x;        // [n] scatter slot -> x (sort key)
     uint4* nbr;            // [(maxnb/8) * npad]
     uint16_t* nnb;         // [npad]
-    double* partial;       // [ntile*4]: pe, ke, virial_abs, virial_pair
+    double* partial;       // [4 parts][ntile][4]: pe, ke, virial_abs, virial_pair (one part: the first),
+                           // then the number of parts the last force launch wrote
     ThermoDev* thermo;     // [thermo_cap]
     const PairParam* pp;   // [ntypes*ntypes]
     const double* mass;    // [ntypes]

@@ -56,11 +56,13 @@ struct Plan {
 pis_status make_plan(const pis_system_desc* d, Plan* p, bool need_types = true);
 // Smallest LDS staging class holding `need` atoms (-1 if none does).
 int stage_class_for(double need);
+// Lanes per atom (1 or 4) of the list-build and force launches over `tiles` tiles.
+int class_lanes(int tiles);
 
 // Offsets of every array of a system's device memory (256-byte aligned) and the total.
 struct Layout {
     size_t st[2][11];
-    size_t r, ctl, cc, cs, n2s, tc, ac, ss, sk, sx, nbr, nnb, part, pp, m, nhc, box, npt, tens;
+    size_t r, ctl, cc, cs, n2s, ac, ss, sk, sx, nbr, nnb, part, pp, m, nhc, box, npt, tens;
     size_t total;
 };
 size_t align256(size_t x);
@@ -101,6 +103,7 @@ struct pis_ctx {
     struct TileClass {
         int scap;
         int kind;  // KIND_* of every tile in the class
+        int lanes; // lanes per atom and workgroups per tile (class_lanes)
         int first;
         int count;
         int lane;  // 0: `stream`, k > 0: side[k-1]

@@ -368,7 +368,9 @@ pis_status plan_grid(Plan* p, double margin)
         p->scap = scap_for(stage * 1.1 + 48);
         if (p->scap < 0) return fail(PIS_ERR_UNSUPPORTED, "tile staging exceeds LDS capacity");
     }
-    p->ntile = p->nt[0] * p->nt[1] * p->nt[2];
+    // a whole-box system's atoms are dealt out kTileThreads at a time, each workgroup staging
+    // the box
+    p->ntile = p->mode == MODE_WHOLE ? (int)((p->n + kTileThreads - 1) / kTileThreads) : p->nt[0] * p->nt[1] * p->nt[2];
     set_bands(p);
     p->npad = (int)((p->n + 63) / 64 * 64);
     int maxnb;
@@ -414,14 +416,13 @@ Layout pis::layout_of(const Plan& p)
     L.cc = take(nc * 4);
     L.cs = take((nc + 1) * 4);
     L.n2s = take(nc * 4);
-    L.tc = take(((size_t)p.ntile + 1) * 4);
     L.ac = take(np * 4);
     L.ss = take(np * 4);
     L.sk = take(np * 4);
     L.sx = take(np * 8);
     L.nbr = take((size_t)(p.maxnb / 8) * np * 16);
     L.nnb = take(np * 2);
-    L.part = take((size_t)p.ntile * 4 * 8);
+    L.part = take(((size_t)p.ntile * 16 + 1) * 8);
     L.pp = take(p.pp.size() * sizeof(PairParam));
     L.m = take(p.mass.size() * 8);
     L.nhc = take(NHC_COUNT * 8);
@@ -435,6 +436,18 @@ Layout pis::layout_of(const Plan& p)
 
 pis_status pis::make_plan(const pis_system_desc* d, Plan* p, bool need_types) { return make_plan_impl(d, p, need_types); }
 int pis::stage_class_for(double need) { return scap_for(need); }
+
+// A launch over few tiles leaves most of the chip's 1024 SIMDs without a wave, and its time is
+// one workgroup's chain of latencies; four lanes per atom and four workgroups per tile cut
+// that chain, for four times the halo staging.  Measured per step, one against four: 500
+// atoms (2 work items) 39 against 26 us, 4000 (18 tiles) 55 against 37, 40 Kob-Andersen
+// systems in classes of 2 to 500 tiles 354 against 288; 176 tiles break even in mixed
+// precision and lose in FP64 (95 against 110 us of an NPT step), 700 tiles lose (65 against
+// 122).  The line lies below the first loss.
+#ifndef PIS_LANES_TILES
+#define PIS_LANES_TILES 128
+#endif
+int pis::class_lanes(int tiles) { return tiles <= PIS_LANES_TILES ? 4 : 1; }
 
 size_t pis::system_bytes(const Plan& p, int thermo_records)
 {
@@ -460,7 +473,6 @@ void pis::carve_system(const Plan& p, const Layout& Lo, char* b, SysDev& d)
     d.cell_count = (int32_t*)(b + Lo.cc);
     d.cell_start = (int32_t*)(b + Lo.cs);
     d.nat2sorted = (int32_t*)(b + Lo.n2s);
-    d.tile_cell0 = (int32_t*)(b + Lo.tc);
     d.atom_cell = (int32_t*)(b + Lo.ac);
     d.scat_src = (int32_t*)(b + Lo.ss);
     d.scat_key = (uint32_t*)(b + Lo.sk);
@@ -527,17 +539,13 @@ pis_status pis::alloc_system(SysHost& h)
     carve_system(p, Lo, (char*)mem, d);
     // zero everything once (outside any captured sequence), then tables
     PIS_HIP(hipMemset(mem, 0, Lo.total));
-    // natural -> sorted (tile-major) cell ids and the first sorted cell of every tile
-    std::vector<int32_t> n2s((size_t)p.ncell), tc((size_t)p.ntile + 1);
+    // natural -> sorted (tile-major) cell ids
+    std::vector<int32_t> n2s((size_t)p.ncell);
     for (int z = 0; z < p.nc[2]; ++z)
         for (int y = 0; y < p.nc[1]; ++y)
             for (int x = 0; x < p.nc[0]; ++x)
                 n2s[((size_t)z * p.nc[1] + y) * p.nc[0] + x] = sorted_cell_id(p.nc, p.tile, x, y, z);
-    for (int t = 0; t < p.ntile; ++t)
-        tc[t] = tile_first_cell(p.nc, p.tile, t % p.nt[0], (t / p.nt[0]) % p.nt[1], t / (p.nt[0] * p.nt[1]));
-    tc[p.ntile] = p.ncell;
     PIS_HIP(hipMemcpy(d.nat2sorted, n2s.data(), n2s.size() * 4, hipMemcpyHostToDevice));
-    PIS_HIP(hipMemcpy(d.tile_cell0, tc.data(), tc.size() * 4, hipMemcpyHostToDevice));
     PIS_HIP(hipMemcpy((void*)d.pp, p.pp.data(), p.pp.size() * sizeof(PairParam), hipMemcpyHostToDevice));
     PIS_HIP(hipMemcpy((void*)d.mass, p.mass.data(), p.mass.size() * 8, hipMemcpyHostToDevice));
     double bx[BOX_COUNT];
@@ -560,18 +568,14 @@ pis_status pis::alloc_system_at(SysHost& h, void* mem, int thermo_records, hipSt
     d.thermo = h.thermo;
     d.thermo_cap = thermo_records;
     PIS_HIP(hipMemsetAsync(mem, 0, Lo.total, st));
-    std::vector<int32_t> n2s((size_t)p.ncell), tc((size_t)p.ntile + 1);
+    std::vector<int32_t> n2s((size_t)p.ncell);
     for (int z = 0; z < p.nc[2]; ++z)
         for (int y = 0; y < p.nc[1]; ++y)
             for (int x = 0; x < p.nc[0]; ++x)
                 n2s[((size_t)z * p.nc[1] + y) * p.nc[0] + x] = sorted_cell_id(p.nc, p.tile, x, y, z);
-    for (int t = 0; t < p.ntile; ++t)
-        tc[t] = tile_first_cell(p.nc, p.tile, t % p.nt[0], (t / p.nt[0]) % p.nt[1], t / (p.nt[0] * p.nt[1]));
-    tc[p.ntile] = p.ncell;
     double bx[BOX_COUNT];
     plan_box(p, bx);
     PIS_HIP(hipMemcpyAsync(d.nat2sorted, n2s.data(), n2s.size() * 4, hipMemcpyHostToDevice, st));
-    PIS_HIP(hipMemcpyAsync(d.tile_cell0, tc.data(), tc.size() * 4, hipMemcpyHostToDevice, st));
     PIS_HIP(hipMemcpyAsync((void*)d.pp, p.pp.data(), p.pp.size() * sizeof(PairParam), hipMemcpyHostToDevice, st));
     PIS_HIP(hipMemcpyAsync((void*)d.mass, p.mass.data(), p.mass.size() * 8, hipMemcpyHostToDevice, st));
     PIS_HIP(hipMemcpyAsync(d.box, bx, sizeof(bx), hipMemcpyHostToDevice, st));
@@ -649,7 +653,8 @@ pis_status pis::group_tiles(pis_ctx* c)
     std::vector<WorkItem> tw;
     c->classes.clear();
     for (auto& kv : by_class) {
-        c->classes.push_back({kv.first.first, kv.first.second, (int)tw.size(), (int)kv.second.size(), 0});
+        const int lanes = class_lanes((int)kv.second.size());
+        c->classes.push_back({kv.first.first, kv.first.second, lanes, (int)tw.size(), (int)kv.second.size(), 0});
         tw.insert(tw.end(), kv.second.begin(), kv.second.end());
     }
     // Classes share up to max_lanes streams (the device serves a few hardware queues per
@@ -877,8 +882,8 @@ pis_status pis::enqueue_classes(pis_ctx* c, bool build, int force)
     }
     for (const auto& q : c->classes) {
         hipStream_t st = q.lane == 0 ? c->stream : c->side[q.lane - 1];
-        if (build) launch_build_list(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, q.kind);
-        if (force >= 0) launch_force(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, c->mixed, force, q.kind);
+        if (build) launch_build_list(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, q.kind, q.lanes);
+        if (force >= 0) launch_force(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, c->mixed, force, q.kind, q.lanes);
     }
     for (int l = 1; l < nl; ++l) {
         PIS_HIP(hipEventRecord(c->join[l - 1], c->side[l - 1]));

@@ -15,11 +15,12 @@ void launch_integrate_pos(hipStream_t st, const SysDev* d_sys, const WorkItem* a
 // Counting sort of every system whose rebuild flag is set (bin, scan, scatter, rank).
 void launch_rebuild_sort(hipStream_t st, const SysDev* d_sys, int nsys, const WorkItem* atom_work,
                          int n_atom_work);
-// Neighbour lists of the tiles of one staging-capacity class.
+// Neighbour lists of the tiles of one staging-capacity class; lanes: lanes per atom and
+// workgroups per tile (1 or 4), the same bits either way.
 void launch_build_list(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work, int n_tile_work,
-                       int scap, int kinds);
+                       int scap, int kinds, int lanes);
 void launch_force(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work,
-                  int n_tile_work, int scap, bool mixed, int integrate, int kinds);
+                  int n_tile_work, int scap, bool mixed, int integrate, int kinds, int lanes);
 // `step` = 1 after an NVE step: frozen systems (ctl[CTL_LEFT] == 0) are skipped and a
 // positive step budget is counted down.
 void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int record, int step);

@@ -228,14 +228,49 @@ __device__ __forceinline__ void wave_runs(int key, bool active, int* head, int* 
 // xcd_remap when REMAP) belongs to a system with its rebuild flag set.  One parallel probe:
 // on steps without a rebuild a block returns after two dependent loads instead of walking
 // its items one by one.
-template <bool REMAP>
+template <bool REMAP, int PARTS = 1>
 __device__ __forceinline__ bool block_rebuild_pending(const SysDev* __restrict__ sys,
                                                       const WorkItem* __restrict__ work, int nwork)
 {
     int flag = 0;
-    for (int b = blockIdx.x + (int)threadIdx.x * (int)gridDim.x; b < nwork; b += (int)(blockDim.x * gridDim.x))
-        flag |= sys[work[REMAP ? xcd_remap(b, nwork) : b].sys].ctl[CTL_REBUILD];
+    const int nb = nwork * PARTS;
+    for (int b = blockIdx.x + (int)threadIdx.x * (int)gridDim.x; b < nb; b += (int)(blockDim.x * gridDim.x))
+        flag |= sys[work[(REMAP ? xcd_remap(b, nb) : b) / PARTS].sys].ctl[CTL_REBUILD];
     return __syncthreads_or(flag) != 0;
+}
+
+// Lane K of each quad's value in all four lanes.
+template <int K>
+__device__ __forceinline__ int quad_bcast(int v)
+{
+    return __builtin_amdgcn_update_dpp(v, v, K * 0x55, 0xF, 0xF, false);
+}
+
+// v of the lane that a DPP control selects (all lanes active).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false));
+}
+
+__device__ __forceinline__ double readlane_f64(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sum over the wave (all lanes active), uniform, in a fixed order: pairs, quads, eights and
+// rows of 16 by DPP, then the four row sums through scalar registers.  A shuffle reduction
+// takes six LDS round trips instead.
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += dpp_f64<0xB1>(v);   // quad_perm [1,0,3,2]
+    v += dpp_f64<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += dpp_f64<0x141>(v);  // row_half_mirror
+    v += dpp_f64<0x140>(v);  // row_mirror
+    return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
 }
 
 // Deterministic sum of 4 doubles over the block (<= 16 waves); result valid in thread 0.
@@ -243,12 +278,7 @@ __device__ void block_sum4(double v[4], double* tmp /* [16 waves * 4] */)
 {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        double x = v[k];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        v[k] = x;
-    }
+    for (int k = 0; k < 4; ++k) v[k] = wave_sum(v[k]);
     if (lane == 0)
         for (int k = 0; k < 4; ++k) tmp[wid * 4 + k] = v[k];
     __syncthreads();
@@ -299,6 +329,7 @@ __device__ __forceinline__ void rel_to_center(const SysDev& s, double cx, double
 __device__ __forceinline__ TileGeom tile_geom(const SysDev& s, int t)
 {
     TileGeom g;
+    if (s.mode == MODE_WHOLE) t = 0;  // every pass stages the whole box
     const int tx = t % s.nt[0], ty = (t / s.nt[0]) % s.nt[1], tz = t / (s.nt[0] * s.nt[1]);
     g.x0 = tx * s.tile[0];
     g.y0 = ty * s.tile[1];
@@ -307,12 +338,53 @@ __device__ __forceinline__ TileGeom tile_geom(const SysDev& s, int t)
     g.sy = min(s.tile[1], s.nc[1] - g.y0);
     g.sz = min(s.tile[2], s.nc[2] - g.z0);
     g.ne = s.mode == MODE_WHOLE ? 1 : (g.sx + 2) * (g.sy + 2) * (g.sz + 2);
-    g.c0 = s.tile_cell0[t];
-    g.c1 = s.tile_cell0[t + 1];
+    // computed, not looked up: one dependent memory round trip less at the start of a tile
+    g.c0 = tile_first_cell(s.nc, s.tile, tx, ty, tz);
+    g.c1 = g.c0 + g.sx * g.sy * g.sz;
     return g;
 }
 
+// Own atoms [a0, a1) of work item t: the tile's cells, or the t-th kTileThreads atoms of a
+// whole-box system.
+__device__ __forceinline__ void own_atoms(const SysDev& s, const TileGeom& g, int t, int* a0, int* a1)
+{
+    if (s.mode == MODE_WHOLE) {
+        *a0 = t * kTileThreads;
+        *a1 = min(s.n, *a0 + kTileThreads);
+    } else {
+        *a0 = gbl(s.cell_start)[g.c0];
+        *a1 = gbl(s.cell_start)[g.c1];
+    }
+}
+
 __device__ __forceinline__ int wrap_cell(int c, int n) { return c < 0 ? c + n : (c >= n ? c - n : c); }
+
+// x / t for 0 <= x <= 1024 and 1 <= t <= 1024, exactly: (x + 1/2) / t lies at least 1 / (2 t)
+// from an integer, and FP32 is off by less than 2^-22 (x + 1/2) / t < 1 / (2 t).
+__device__ __forceinline__ int cell_div(int x, int t)
+{
+    return (int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)t));
+}
+
+// sorted_cell_id (common.h) without integer division, instead of a look-up in nat2sorted: a
+// memory round trip less before a tile's cells are known.
+__device__ __forceinline__ int sorted_cell(const SysDev& s, int x, int y, int z)
+{
+    const int tx = cell_div(x, s.tile[0]), ty = cell_div(y, s.tile[1]), tz = cell_div(z, s.tile[2]);
+    const int sx = min(s.tile[0], s.nc[0] - tx * s.tile[0]), sy = min(s.tile[1], s.nc[1] - ty * s.tile[1]);
+    return tile_first_cell(s.nc, s.tile, tx, ty, tz) + ((z - tz * s.tile[2]) * sy + (y - ty * s.tile[1])) * sx +
+           (x - tx * s.tile[0]);
+}
+
+// Sorted id of halo cell e (x fastest) of a tile.
+__device__ __forceinline__ int halo_cell(const SysDev& s, const TileGeom& g, int e)
+{
+    const int hx = g.sx + 2, hy = g.sy + 2;
+    const int row = cell_div(e, hx), ez = cell_div(row, hy);
+    const int ex = e - row * hx, ey = row - ez * hy;
+    return sorted_cell(s, wrap_cell(g.x0 - 1 + ex, s.nc[0]), wrap_cell(g.y0 - 1 + ey, s.nc[1]),
+                       wrap_cell(g.z0 - 1 + ez, s.nc[2]));
+}
 
 enum { STAGE_RAW = 0, STAGE_REL = 1, STAGE_INDEX = 2 };
 constexpr double kPadFar = 1e30;  // squared: 1e60, finite in FP64, +inf in FP32
@@ -328,7 +400,7 @@ constexpr double kPadFar = 1e30;  // squared: 1e60, finite in FP64, +inf in FP32
 // every slot, each cell's thread filling its run, so a slot finds its atom with one LDS
 // read instead of a binary search over the halo's cell offsets.  Staged coordinates are
 // multiplied by `scale` (1, or 1/sigma for the single-species mixed loop).
-template <int SCAP, int WHAT, typename T>
+template <int SCAP, int WHAT, typename T, bool WIDE = false>
 __device__ int stage_tile(const SysDev& s, const State& st, const TileGeom& g, double cx, double cy,
                           double cz, T* Px, T* Py, T* Pz, uint8_t* Pt, int* pref, int* ecell, int* stmp,
                           uint8_t* smap = nullptr, double scale = 1.0)
@@ -342,12 +414,7 @@ __device__ int stage_tile(const SysDev& s, const State& st, const TileGeom& g, d
             cnt = s.n;
         }
     } else if (tid < ne) {
-        const int hx = g.sx + 2, hy = g.sy + 2;
-        const int ex = tid % hx, ey = (tid / hx) % hy, ez = tid / (hx * hy);
-        const int cxn = wrap_cell(g.x0 - 1 + ex, s.nc[0]);
-        const int cyn = wrap_cell(g.y0 - 1 + ey, s.nc[1]);
-        const int czn = wrap_cell(g.z0 - 1 + ez, s.nc[2]);
-        const int sc = gbl(s.nat2sorted)[(czn * s.nc[1] + cyn) * s.nc[0] + cxn];
+        const int sc = halo_cell(s, g, tid);
         const int b = gbl(s.cell_start)[sc];
         ecell[tid] = b;
         cnt = gbl(s.cell_start)[sc + 1] - b;
@@ -358,13 +425,57 @@ __device__ int stage_tile(const SysDev& s, const State& st, const TileGeom& g, d
     if (tid == 0) pref[ne] = total;
     __syncthreads();
     if (total > SCAP) return total;
+    int total_staged = 0;
+    if constexpr (WIDE) {
+        // a half-wave per halo cell, every cell of a round in flight: no slot-to-cell map to
+        // fill and to search, at the price of idle lanes (a cell holds 19 to 32 atoms)
+        if (ne > 1) {
+            constexpr int R = 5;
+            const int nh = (int)blockDim.x >> 5, h = tid >> 5, l = tid & 31;
+            for (int e0 = h; e0 < ne; e0 += R * nh) {
+                double x[R], y[R], z[R];
+                uint8_t ty[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int e = e0 + r * nh;
+                    if (e >= ne || l >= pref[e + 1] - pref[e]) continue;
+                    const int a = ecell[e] + l;
+                    x[r] = gbl(st.x)[a];
+                    y[r] = gbl(st.y)[a];
+                    z[r] = gbl(st.z)[a];
+                    ty[r] = Pt ? gbl(st.type)[a] : 0;
+                }
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int e = e0 + r * nh;
+                    if (e >= ne) break;
+                    const int p0 = pref[e], n = pref[e + 1] - p0;
+                    for (int i = l; i < n; i += 32) {
+                        if (i != l) {  // a cell of more than 32 atoms
+                            const int a = ecell[e] + i;
+                            x[r] = gbl(st.x)[a];
+                            y[r] = gbl(st.y)[a];
+                            z[r] = gbl(st.z)[a];
+                            ty[r] = Pt ? gbl(st.type)[a] : 0;
+                        }
+                        if (WHAT == STAGE_REL) rel_to_center(s, cx, cy, cz, x[r], y[r], z[r]);
+                        Px[p0 + i] = (T)(x[r] * scale);
+                        Py[p0 + i] = (T)(y[r] * scale);
+                        Pz[p0 + i] = (T)(z[r] * scale);
+                        if (Pt) Pt[p0 + i] = ty[r];
+                    }
+                }
+            }
+            total_staged = total;
+        }
+    }
     const bool mapped = smap != nullptr && ne > 1;
     if (mapped) {
         if (tid < ne)
             for (int sl = ex; sl < ex + cnt; ++sl) smap[sl] = (uint8_t)tid;
         __syncthreads();
     }
-    for (int sl = tid; sl < total; sl += blockDim.x) {
+    for (int sl = total_staged + tid; sl < total; sl += blockDim.x) {
         int lo = 0;
         if (mapped) {
             lo = smap[sl];
@@ -905,7 +1016,7 @@ __device__ __forceinline__ lds_cf32* lds_opaque(const float* p)
 // shift register that leaves as one uint4 list group per 8 entries.  r2 from the staged
 // coordinates decides every pair outside a +-band around the cutoff; inside the band the
 // bit-exact reference predicate (exact_within, raw positions) decides.
-template <int SCAP, bool PAIRMI, int NT, bool TRI>
+template <int SCAP, bool PAIRMI, int NT, bool TRI, int KL>
 __device__ __forceinline__ int build_atom(const SysDev& s, const State& st, const TileGeom& g,
                                           const float* Px, const float* Py, const float* Pz,
                                           const uint8_t* Pt, const int* pref, const int* ecell,
@@ -1025,6 +1136,106 @@ __device__ __forceinline__ int build_atom(const SysDev& s, const State& st, cons
         ++cnt;
         if ((cnt & 7) == 0 && (cnt >> 3) <= maxg) out[(size_t)((cnt >> 3) - 1) * npad] = u32x4{w0, w1, w2, w3};
     };
+    // the per-pair image of raw staging, this lane's list-band edges against a partner type,
+    // and the reference predicate for a candidate inside the band
+    auto image = [&](float& dx, float& dy, float& dz) {
+        if (PAIRMI && TRI) {
+            mi_tri32(H32, HI32, dx, dy, dz);
+        } else if (PAIRMI) {
+            dx = mi_fast32(dx, L32[0], Li32[0]);
+            dy = mi_fast32(dy, L32[1], Li32[1]);
+            dz = mi_fast32(dz, L32[2], Li32[2]);
+        }
+    };
+    auto edges = [&](int tt, float& blo, float& bhi) {
+        blo = tlo[0];
+        bhi = thi[0];
+        if (NT == 2) {  // one select per edge: the partner is type 0 or 1
+            blo = tt != 0 ? tlo[1] : blo;
+            bhi = tt != 0 ? thi[1] : bhi;
+        } else if (MULTI) {
+            blo = tt == 1 ? tlo[1] : blo;
+            bhi = tt == 1 ? thi[1] : bhi;
+            blo = tt == 2 ? tlo[2] : blo;
+            bhi = tt == 2 ? thi[2] : bhi;
+            blo = tt == 3 ? tlo[3] : blo;
+            bhi = tt == 3 ? thi[3] : bhi;
+        }
+    };
+    auto settle = [&](int sl) {
+        const PairParam& p = ppl[MULTI ? ti * nt + Pt[sl] : 0];
+        return exact_within<TRI>(s, st, slot_atom(pref, ecell, g.ne, sl), xi, yi, zi, p.r2_list);
+    };
+    if constexpr (KL > 1) {
+        // Four lanes per atom take 8 candidates each of a 32-candidate block of a row (the
+        // quad's lanes share the atom and so the rows, in the order the single lane takes
+        // them); the lanes' accepted counts give each its place in the list, and entries are
+        // stored one by one (2 bytes), since a group of 8 has up to four writers.
+        const int sub = (int)threadIdx.x % KL;
+        __attribute__((address_space(1))) uint16_t* out16 = gbl(reinterpret_cast<uint16_t*>(s.nbr + a));
+        auto store = [&](int pos, uint32_t entry) {
+            if ((pos >> 3) < maxg) out16[(size_t)(pos >> 3) * npad * 8 + (pos & 7)] = (uint16_t)entry;
+        };
+        for (int r = 0; r < nrows; ++r) {
+            const int rb = (int)(key[0] & 0xffffu), re = rb + (int)(key[0] >> 16);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) key[q] = key[q + 1];
+            key[8] = 0u;
+            const int rowmax = wave_max(re - rb);
+            for (int cb = 0; cb < rowmax; cb += 8 * KL) {
+                const int sb = rb + cb + 8 * sub;
+                const int sr = sb < re ? sb : 0;  // a used-up window reads slot 0 onwards
+                lds_cf32* px = lds_opaque(Px + sr);
+                lds_cf32* py = lds_opaque(Py + sr);
+                lds_cf32* pz = lds_opaque(Pz + sr);
+                float dx[8], dy[8], dz[8];
+                int tt[8];
+                uint32_t mi = 0, mm = 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    dx[j] = px[j] - qx32;
+                    dy[j] = py[j] - qy32;
+                    dz[j] = pz[j] - qz32;
+                    tt[j] = MULTI ? (int)Pt[sr + j] : 0;
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    image(dx[j], dy[j], dz[j]);
+                    const float r2 = fmaf(dx[j], dx[j], fmaf(dy[j], dy[j], dz[j] * dz[j]));
+                    float blo, bhi;
+                    edges(tt[j], blo, bhi);
+                    shift_in_le(mi, r2, blo);
+                    shift_in_le(mm, r2, bhi);
+                }
+                mi = __builtin_bitreverse32(mi) >> 24;
+                mm = __builtin_bitreverse32(mm) >> 24;
+                const int nv = max(0, min(8, re - sb)), ds = self - sb;
+                uint32_t keep = (1u << nv) - 1u;  // inside the window, not the atom itself
+                if (ds >= 0 && ds < 8) keep &= ~(1u << ds);
+                uint32_t m = mi & keep, bm = mm & ~mi & keep;
+                if (__any(bm != 0u)) {
+                    while (bm) {
+                        const int k = __builtin_ctz(bm);
+                        bm &= bm - 1u;
+                        if (settle(sb + k)) m |= 1u << k;
+                    }
+                }
+                const int n = __builtin_popcount(m);
+                const int n0 = quad_bcast<0>(n), n1 = quad_bcast<1>(n), n2 = quad_bcast<2>(n), n3 = quad_bcast<3>(n);
+                int pos = cnt + (sub > 0 ? n0 : 0) + (sub > 1 ? n1 : 0) + (sub > 2 ? n2 : 0);
+                cnt += (n0 + n1) + (n2 + n3);
+                while (m) {
+                    const uint32_t sl = (uint32_t)(sb + __builtin_ctz(m));
+                    m &= m - 1u;
+                    store(pos++, (sl << lsh) | (MULTI ? (uint32_t)Pt[sl] : 0u));
+                }
+            }
+        }
+        if (!active) return 0;
+        for (int pos = cnt + sub; pos < ((cnt + 7) & ~7); pos += KL) store(pos, (uint32_t)SCAP << lsh);
+        if (sub == 0) gbl(s.nnb)[a] = (uint16_t)min(cnt, s.maxnb);
+        return cnt;
+    }
     for (int r = 0; r < nrows; ++r) {
         const int rb = (int)(key[0] & 0xffffu), re = rb + (int)(key[0] >> 16);
 #pragma unroll
@@ -1061,26 +1272,10 @@ __device__ __forceinline__ int build_atom(const SysDev& s, const State& st, cons
                     }
 #pragma unroll
                     for (int j = 0; j < U; ++j) {
-                        if (PAIRMI && TRI) {
-                            mi_tri32(H32, HI32, dx[j], dy[j], dz[j]);
-                        } else if (PAIRMI) {
-                            dx[j] = mi_fast32(dx[j], L32[0], Li32[0]);
-                            dy[j] = mi_fast32(dy[j], L32[1], Li32[1]);
-                            dz[j] = mi_fast32(dz[j], L32[2], Li32[2]);
-                        }
+                        image(dx[j], dy[j], dz[j]);
                         const float r2 = fmaf(dx[j], dx[j], fmaf(dy[j], dy[j], dz[j] * dz[j]));
-                        float blo = tlo[0], bhi = thi[0];
-                        if (NT == 2) {  // one select per edge: the partner is type 0 or 1
-                            blo = tt[j] != 0 ? tlo[1] : blo;
-                            bhi = tt[j] != 0 ? thi[1] : bhi;
-                        } else if (MULTI) {
-                            blo = tt[j] == 1 ? tlo[1] : blo;
-                            bhi = tt[j] == 1 ? thi[1] : bhi;
-                            blo = tt[j] == 2 ? tlo[2] : blo;
-                            bhi = tt[j] == 2 ? thi[2] : bhi;
-                            blo = tt[j] == 3 ? tlo[3] : blo;
-                            bhi = tt[j] == 3 ? thi[3] : bhi;
-                        }
+                        float blo, bhi;
+                        edges(tt[j], blo, bhi);
                         if (PIS_BUILD_SHIFTIN) {  // candidate k0 + i ends at bit n - 1 - i
                             shift_in_le(mi, r2, blo);
                             shift_in_le(mm, r2, bhi);
@@ -1124,9 +1319,7 @@ __device__ __forceinline__ int build_atom(const SysDev& s, const State& st, cons
                     while (bm) {
                         const int kk = __builtin_ctz(bm) + 32 * half;
                         bm &= bm - 1u;
-                        const int sl = sb + kk;
-                        const PairParam& p = ppl[MULTI ? ti * nt + Pt[sl] : 0];
-                        if (exact_within<TRI>(s, st, slot_atom(pref, ecell, g.ne, sl), xi, yi, zi, p.r2_list)) {
+                        if (settle(sb + kk)) {
                             if (kk < 32)
                                 mlo |= 1u << kk;
                             else
@@ -1172,7 +1365,7 @@ __device__ __forceinline__ int system_kind(const SysDev& s)
 
 // One instantiation per kind (KIND_*), so the common tile-relative kinds carry neither the
 // per-pair image of raw staging nor its registers.
-template <int SCAP, int KIND>
+template <int SCAP, int KIND, int KL>
 __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_list(const SysDev* __restrict__ sys,
                                                               const WorkItem* __restrict__ tiles,
                                                               int ntw)
@@ -1191,9 +1384,10 @@ __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_lis
     __shared__ uint16_t wtab[(kMaxHalo + 1) * kWinSlices];  // row-window table (orthorhombic, tile-relative)
     __shared__ int ownf[kMaxHalo];  // first atom of each own cell
     const int lane = threadIdx.x & 63;
-    if (!block_rebuild_pending<true>(sys, tiles, ntw)) return;
-    for (int b = blockIdx.x; b < ntw; b += gridDim.x) {
-        const WorkItem w = tiles[xcd_remap(b, ntw)];
+    if (!block_rebuild_pending<true, KL>(sys, tiles, ntw)) return;
+    for (int b = blockIdx.x; b < ntw * KL; b += gridDim.x) {
+        const int item = xcd_remap(b, ntw * KL), part = item % KL;
+        const WorkItem w = tiles[item / KL];
         const SysDev& s = sys[w.sys];
         if (!s.ctl[CTL_REBUILD]) continue;
         if (system_kind(s) != KIND) continue;  // another instantiation builds this tile
@@ -1203,8 +1397,8 @@ __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_lis
         double cx, cy, cz;
         tile_center(s, g, cx, cy, cz);
         for (int q = threadIdx.x; q < nt * nt; q += blockDim.x) ppl[q] = s.pp[q];
-        const int total = stage_tile<SCAP, REL ? STAGE_REL : STAGE_RAW>(s, st, g, cx, cy, cz, Px, Py, Pz, Pt, pref,
-                                                                          ecell, stmp, smap);
+        const int total = stage_tile<SCAP, REL ? STAGE_REL : STAGE_RAW, float, (KL > 1)>(
+            s, st, g, cx, cy, cz, Px, Py, Pz, Pt, pref, ecell, stmp, smap);
         if (threadIdx.x == 0) atomicMax(&s.ctl[CTL_MAXSTAGE], total);
         if (total > SCAP) {
             if (threadIdx.x == 0) atomicOr(&s.ctl[CTL_OVF_STAGE], 1);
@@ -1245,22 +1439,24 @@ __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_lis
         } else {
             __syncthreads();
         }
-        const int a0 = s.cell_start[g.c0], a1 = s.cell_start[g.c1];
+        int a0, a1;
+        own_atoms(s, g, w.idx, &a0, &a1);
         int mymax = 0;
         // whole waves iterate together (inactive lanes ride along) so the sweeps stay uniform
-        const int span = ((a1 - a0) + 63) & ~63;
-        for (int base = a0 + (int)(threadIdx.x & ~63); base < a0 + span; base += blockDim.x) {
-            const int a = base + lane;
+        // a wave's 64 / KL atoms; with four lanes per atom this workgroup is one of the four parts
+        // of the tile: 64 of every 256 of its atoms
+        for (int base = a0 + part * 64 + (int)(threadIdx.x / 64) * (64 / KL); base < a1; base += kTileThreads) {
+            const int a = base + lane / KL;
             const bool active = a < a1;
             // REL: tile-relative staging (plain differences); otherwise raw positions and the
             // per-pair image of the box
             const int n =
-                nt == 1   ? build_atom<SCAP, !REL, 1, TRI>(s, st, g, Px, Py, Pz, Pt, pref, ecell, ownf, ppl, wtab,
-                                                           total, active, a, cx, cy, cz)
-                : nt == 2 ? build_atom<SCAP, !REL, 2, TRI>(s, st, g, Px, Py, Pz, Pt, pref, ecell, ownf, ppl, wtab,
-                                                           total, active, a, cx, cy, cz)
-                          : build_atom<SCAP, !REL, kMaxTypes, TRI>(s, st, g, Px, Py, Pz, Pt, pref, ecell, ownf,
-                                                                   ppl, wtab, total, active, a, cx, cy, cz);
+                nt == 1   ? build_atom<SCAP, !REL, 1, TRI, KL>(s, st, g, Px, Py, Pz, Pt, pref, ecell, ownf, ppl, wtab,
+                                                               total, active, a, cx, cy, cz)
+                : nt == 2 ? build_atom<SCAP, !REL, 2, TRI, KL>(s, st, g, Px, Py, Pz, Pt, pref, ecell, ownf, ppl, wtab,
+                                                               total, active, a, cx, cy, cz)
+                          : build_atom<SCAP, !REL, kMaxTypes, TRI, KL>(s, st, g, Px, Py, Pz, Pt, pref, ecell, ownf,
+                                                                       ppl, wtab, total, active, a, cx, cy, cz);
             mymax = max(mymax, n);
         }
         mymax = wave_max(mymax);
@@ -1278,50 +1474,80 @@ __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_lis
 struct Acc {
     double fx, fy, fz, pe, wp;
 };
+struct Acc32 {
+    float fx, fy, fz, pe, wp;
+};
 
 // LennardJones::compute_potential (lennard_jones.rs:32-55) for one candidate, without a
-// branch: `in` selects whether the pair contributes.  FP64: a refined hardware reciprocal
-// for 1/r2; a candidate outside the cutoff computes with its own finite r2 and is dropped
-// by the selects (raw staging masks padding entries by count, tile-relative staging puts
-// the padding slot kPadFar away, so its r2 is finite in FP64 and fails the cutoff).  MIXED
-// with FP64 staging (raw staging only): r2 and the cutoff decision stay FP64, the LJ
-// arithmetic is FP32, and a candidate outside the cutoff enters it as r2 = +inf, which
-// v_rcp_f32 turns into +0 (force factor -0; the energy shift is masked to 0).  Results
-// accumulate in FP64.
-template <bool MIXED>
-__device__ __forceinline__ void lj_accum(const PairParam& p, double dx, double dy, double dz, double r2,
-                                         bool in, Acc& acc)
+// branch: `in` selects whether the pair contributes.
+//
+// FP64: 1/r^2 from the hardware reciprocal (about 2^-23 off, e its residual) and one
+// third-order step, inv (1 + e + e^2): three FMAs to full precision, where two Newton steps
+// take four.  It is zeroed for a candidate outside the cutoff (raw staging masks padding
+// entries by count, tile-relative staging puts the padding slot kPadFar away, so its r^2 is
+// finite in FP64 and fails the cutoff), and every power and product of it is then zero.
+__device__ __forceinline__ double masked_inverse(double r2, bool in)
 {
-    if (!MIXED) {
-        double inv = __builtin_amdgcn_rcp(r2);
-        inv = fma(inv, fma(-r2, inv, 1.0), inv);
-        inv = fma(inv, fma(-r2, inv, 1.0), inv);
-        const double sr2 = p.sig2 * inv;
-        const double sr6 = sr2 * sr2 * sr2;
-        const double fp = in ? fma(p.c48, sr6, -p.c24) * sr6 * inv : 0.0;
-        const double u = in ? fma(fma(p.c4, sr6, -p.c4), sr6, -p.ucut) : 0.0;
-        acc.fx = fma(-fp, dx, acc.fx);
-        acc.fy = fma(-fp, dy, acc.fy);
-        acc.fz = fma(-fp, dz, acc.fz);
-        acc.pe += u;
-        acc.wp = fma(fp, r2, acc.wp);
-    } else {
-        // one 32-bit select each for r2 and the shift, ahead of the FP64 conversions,
-        // instead of two per 64-bit result
-        const float r2f = in ? (float)r2 : __builtin_inff();
-        const float inv = __builtin_amdgcn_rcpf(r2f);
-        const float sr2 = p.sig2f * inv;
-        const float sr6 = sr2 * sr2 * sr2;
-        const float fpf = fmaf(p.c48f, sr6, -p.c24f) * sr6 * inv;
-        const float ucf = in ? p.ucutf : 0.0f;
-        const float uf = fmaf(fmaf(p.c4f, sr6, -p.c4f), sr6, -ucf);
-        const double fp = (double)fpf;
-        acc.fx = fma(-fp, dx, acc.fx);
-        acc.fy = fma(-fp, dy, acc.fy);
-        acc.fz = fma(-fp, dz, acc.fz);
-        acc.pe += (double)uf;
-        acc.wp = fma(fp, r2, acc.wp);
-    }
+    const double x = __builtin_amdgcn_rcp(r2);
+    const double e = fma(-r2, x, 1.0);
+    const double inv = fma(x, fma(e, e, e), x);
+    return in ? inv : 0.0;
+}
+
+// One species: the sums of (sigma/r)^12 (in acc.pe), (sigma/r)^6 (in acc.wp) and the number of
+// pairs in range stand for the energy and the virial (finish_one_species): 3 operations per
+// entry for them instead of 6.
+__device__ __forceinline__ void lj_accum_one(const PairParam& p, double dx, double dy, double dz, double r2, bool in,
+                                             Acc& acc, uint32_t& nin)
+{
+    const double inv = masked_inverse(r2, in);
+    const double sr2 = p.sig2 * inv;
+    const double sr6 = sr2 * sr2 * sr2;
+    const double fp = fma(p.c48, sr6, -p.c24) * sr6 * inv;
+    acc.fx = fma(-fp, dx, acc.fx);
+    acc.fy = fma(-fp, dy, acc.fy);
+    acc.fz = fma(-fp, dz, acc.fz);
+    acc.pe = fma(sr6, sr6, acc.pe);
+    acc.wp += sr6;
+    nin += in ? 1u : 0u;
+}
+
+__device__ __forceinline__ void lj_accum(const PairParam& p, double dx, double dy, double dz, double r2, bool in,
+                                         Acc& acc)
+{
+    const double inv = masked_inverse(r2, in);
+    const double sr2 = p.sig2 * inv;
+    const double sr6 = sr2 * sr2 * sr2;
+    const double w = fma(p.c48, sr6, -p.c24) * sr6;
+    const double fp = w * inv;
+    acc.fx = fma(-fp, dx, acc.fx);
+    acc.fy = fma(-fp, dy, acc.fy);
+    acc.fz = fma(-fp, dz, acc.fz);
+    acc.pe += fma(fma(p.c4, sr6, -p.c4), sr6, -(in ? p.ucut : 0.0));
+    acc.wp += w;
+}
+
+// Mixed precision with FP64 staging (raw staging only): r^2 and the cutoff decision stay
+// FP64, the LJ arithmetic is FP32, and a candidate outside the cutoff enters it as r^2 =
+// +inf, which v_rcp_f32 turns into +0 (force factor -0; the energy shift is masked to 0):
+// one 32-bit select each for r^2 and the shift instead of two per 64-bit result.  Results
+// accumulate in FP64.
+__device__ __forceinline__ void lj_accum_mixed(const PairParam& p, double dx, double dy, double dz, double r2, bool in,
+                                               Acc& acc)
+{
+    const float r2f = in ? (float)r2 : __builtin_inff();
+    const float inv = __builtin_amdgcn_rcpf(r2f);
+    const float sr2 = p.sig2f * inv;
+    const float sr6 = sr2 * sr2 * sr2;
+    const float fpf = fmaf(p.c48f, sr6, -p.c24f) * sr6 * inv;
+    const float ucf = in ? p.ucutf : 0.0f;
+    const float uf = fmaf(fmaf(p.c4f, sr6, -p.c4f), sr6, -ucf);
+    const double fp = (double)fpf;
+    acc.fx = fma(-fp, dx, acc.fx);
+    acc.fy = fma(-fp, dy, acc.fy);
+    acc.fz = fma(-fp, dz, acc.fz);
+    acc.pe += (double)uf;
+    acc.wp = fma(fp, r2, acc.wp);
 }
 
 struct ExactCtx {
@@ -1335,85 +1561,150 @@ struct ExactCtx {
 
 typedef __attribute__((address_space(1))) const u32x4 gu32x4;
 
-template <int SCAP, bool MIXED, bool MULTI, bool PAIRMI, bool TRI>
-__device__ __forceinline__ void atom_forces(const SysDev& s, const double* Px, const double* Py,
-                                            const double* Pz,
-                                            const PairParam* ppl, const PairParam& p0, int a, int ti,
-                                            double qx, double qy, double qz, const ExactCtx& ex,
-                                            Acc& acc)
+template <int K>
+__device__ __forceinline__ double quad_bcast(double v)
 {
-    const int nn = gbl(s.nnb)[a];
-    const int ng = (nn + 7) >> 3;
-    const gu32x4* L = (const gu32x4*)(s.nbr + a);
+    return __hiloint2double(quad_bcast<K>(__double2hiint(v)), quad_bcast<K>(__double2loint(v)));
+}
+template <int K>
+__device__ __forceinline__ float quad_bcast(float v)
+{
+    return __int_as_float(quad_bcast<K>(__float_as_int(v)));
+}
+
+// Lane K's sums added into the accumulators of all four lanes.
+template <int K>
+__device__ __forceinline__ void quad_add(Acc& acc, const Acc& t)
+{
+    acc.fx += quad_bcast<K>(t.fx);
+    acc.fy += quad_bcast<K>(t.fy);
+    acc.fz += quad_bcast<K>(t.fz);
+    acc.pe += quad_bcast<K>(t.pe);
+    acc.wp += quad_bcast<K>(t.wp);
+}
+template <int K>
+__device__ __forceinline__ void quad_add(Acc& acc, const Acc32& t)
+{
+    acc.fx += (double)quad_bcast<K>(t.fx);
+    acc.fy += (double)quad_bcast<K>(t.fy);
+    acc.fz += (double)quad_bcast<K>(t.fz);
+    acc.pe += (double)quad_bcast<K>(t.pe);
+    acc.wp += (double)quad_bcast<K>(t.wp);
+}
+
+// An atom's list, group by group: group(g, u, nin) returns the sums of group g (its 8 entries
+// in u; nin counts pairs in range), and the groups' sums are added into acc in list order.
+// KL = 1: one lane takes every group.  KL = 4: the quad's lanes take a group each and all add
+// the four in order, so the result does not depend on how many lanes an atom was given.  un:
+// the lane's first group (requested by the caller); the next is requested a round ahead.
+template <int KL, class F>
+__device__ __forceinline__ void sum_list(const gu32x4* L, size_t npad, int ng, u32x4 un, Acc& acc, uint32_t& nin,
+                                         F&& group)
+{
+    if constexpr (KL == 1) {
+        for (int g = 0; g < ng; ++g) {
+            const u32x4 u = un;
+            if (g + 1 < ng) un = L[(size_t)(g + 1) * npad];
+            const auto t = group(g, u, nin);
+            acc.fx += (double)t.fx;
+            acc.fy += (double)t.fy;
+            acc.fz += (double)t.fz;
+            acc.pe += (double)t.pe;
+            acc.wp += (double)t.wp;
+        }
+    } else {
+        const int sub = (int)threadIdx.x % KL;
+        for (int g0 = 0; g0 < ng; g0 += KL) {  // uniform over the quad
+            const u32x4 u = un;
+            const int g = g0 + sub;
+            if (g + KL < ng) un = L[(size_t)(g + KL) * npad];
+            decltype(group(g, u, nin)) t = {};
+            if (g < ng) t = group(g, u, nin);
+            quad_add<0>(acc, t);
+            if (g0 + 1 < ng) quad_add<1>(acc, t);
+            if (g0 + 2 < ng) quad_add<2>(acc, t);
+            if (g0 + 3 < ng) quad_add<3>(acc, t);
+        }
+        nin = quad_bcast<0>((int)nin) + quad_bcast<1>((int)nin) + quad_bcast<2>((int)nin) + quad_bcast<3>((int)nin);
+    }
+}
+
+// Sums of list group g (entries u) of an atom with FP64 staging.
+template <int SCAP, bool MIXED, bool MULTI, bool PAIRMI, bool TRI>
+__device__ __forceinline__ Acc group_f64(const SysDev& s, const double* Px, const double* Py, const double* Pz,
+                                         const PairParam* ppl, const PairParam& p0, int g, u32x4 u, int nn, int ti,
+                                         double qx, double qy, double qz, const ExactCtx& ex, uint32_t& nin)
+{
     const char* bx = reinterpret_cast<const char*>(Px);
     const char* by = reinterpret_cast<const char*>(Py);
     const char* bz = reinterpret_cast<const char*>(Pz);
-    u32x4 un = {0u, 0u, 0u, 0u};
-    if (ng > 0) un = L[0];
-    for (int gi = 0; gi < ng; ++gi) {
-        const u32x4 u = un;
-        if (gi + 1 < ng) un = L[(size_t)(gi + 1) * s.npad];
-        const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
-        const int rem = nn - gi * 8;
+    Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
+    const int rem = nn - g * 8;
 #pragma unroll
-        for (int h = 0; h < 8; h += PIS_FORCE_BATCH) {
-            constexpr int B = PIS_FORCE_BATCH;
-            uint32_t off[B];
-            double X[B], Y[B], Z[B];
+    for (int h = 0; h < 8; h += PIS_FORCE_BATCH) {
+        constexpr int B = PIS_FORCE_BATCH;
+        uint32_t off[B];
+        double X[B], Y[B], Z[B];
 #pragma unroll
-            for (int e = 0; e < B; ++e) {
-                const int k = h + e;
-                off[e] = (wv[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
-                const uint32_t ad = MULTI ? off[e] & ~7u : off[e];  // low bits: partner type
-                X[e] = *reinterpret_cast<const double*>(bx + ad);
-                Y[e] = *reinterpret_cast<const double*>(by + ad);
-                Z[e] = *reinterpret_cast<const double*>(bz + ad);
+        for (int e = 0; e < B; ++e) {
+            const int k = h + e;
+            off[e] = (wv[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+            const uint32_t ad = MULTI ? off[e] & ~7u : off[e];  // low bits: partner type
+            X[e] = *reinterpret_cast<const double*>(bx + ad);
+            Y[e] = *reinterpret_cast<const double*>(by + ad);
+            Z[e] = *reinterpret_cast<const double*>(bz + ad);
+        }
+        double R2[B];
+        bool IN[B];
+        bool band = false;
+#pragma unroll
+        for (int e = 0; e < B; ++e) {
+            double dx = X[e] - qx, dy = Y[e] - qy, dz = Z[e] - qz;
+            if (PAIRMI && TRI) {
+                mi_tri_fast(s.box, dx, dy, dz);
+            } else if (PAIRMI) {
+                dx = mi_fast(dx, s.L[0], s.Linv[0]);
+                dy = mi_fast(dy, s.L[1], s.Linv[1]);
+                dz = mi_fast(dz, s.L[2], s.Linv[2]);
             }
-            double R2[B];
-            bool IN[B];
-            bool band = false;
-#pragma unroll
-            for (int e = 0; e < B; ++e) {
-                double dx = X[e] - qx, dy = Y[e] - qy, dz = Z[e] - qz;
-                if (PAIRMI && TRI) {
-                    mi_tri_fast(s.box, dx, dy, dz);
-                } else if (PAIRMI) {
-                    dx = mi_fast(dx, s.L[0], s.Linv[0]);
-                    dy = mi_fast(dy, s.L[1], s.Linv[1]);
-                    dz = mi_fast(dz, s.L[2], s.Linv[2]);
-                }
-                X[e] = dx;
-                Y[e] = dy;
-                Z[e] = dz;
-                R2[e] = fma(dx, dx, fma(dy, dy, dz * dz));
-                const PairParam& p = MULTI ? ppl[ti * s.ntypes + (off[e] & 7u)] : p0;
-                // tile-relative staging: padding entries fail the cutoff by distance
-                const bool valid = PAIRMI ? h + e < rem : true;
-                if (MIXED) {
-                    IN[e] = valid && R2[e] <= p.r2_force;
-                } else {
-                    IN[e] = valid && R2[e] <= p.f_lo;
-                    band |= valid && !IN[e] && R2[e] <= p.f_hi;
-                }
-            }
-            if (!MIXED && band) {
-                // the reference's `norm() > rcut` settled exactly inside the rounding band
-#pragma unroll
-                for (int e = 0; e < B; ++e) {
-                    const PairParam& p = MULTI ? ppl[ti * s.ntypes + (off[e] & 7u)] : p0;
-                    if ((!PAIRMI || h + e < rem) && !IN[e] && R2[e] <= p.f_hi)
-                        IN[e] = exact_within<TRI>(*ex.s, *ex.st,
-                                             slot_atom(ex.pref, ex.ecell, ex.ne, (int)(off[e] >> 3)), ex.xi,
-                                             ex.yi, ex.zi, p.r2_force);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < B; ++e) {
-                const PairParam& p = MULTI ? ppl[ti * s.ntypes + (off[e] & 7u)] : p0;
-                lj_accum<MIXED>(p, X[e], Y[e], Z[e], R2[e], IN[e], acc);
+            X[e] = dx;
+            Y[e] = dy;
+            Z[e] = dz;
+            R2[e] = fma(dx, dx, fma(dy, dy, dz * dz));
+            const PairParam& p = MULTI ? ppl[ti * s.ntypes + (off[e] & 7u)] : p0;
+            // tile-relative staging: padding entries fail the cutoff by distance
+            const bool valid = PAIRMI ? h + e < rem : true;
+            if (MIXED) {
+                IN[e] = valid && R2[e] <= p.r2_force;
+            } else {
+                IN[e] = valid && R2[e] <= p.f_lo;
+                band |= valid && !IN[e] && R2[e] <= p.f_hi;
             }
         }
+        if (!MIXED && band) {
+            // the reference's `norm() > rcut` settled exactly inside the rounding band
+#pragma unroll
+            for (int e = 0; e < B; ++e) {
+                const PairParam& p = MULTI ? ppl[ti * s.ntypes + (off[e] & 7u)] : p0;
+                if ((!PAIRMI || h + e < rem) && !IN[e] && R2[e] <= p.f_hi)
+                    IN[e] = exact_within<TRI>(*ex.s, *ex.st,
+                                         slot_atom(ex.pref, ex.ecell, ex.ne, (int)(off[e] >> 3)), ex.xi,
+                                         ex.yi, ex.zi, p.r2_force);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < B; ++e) {
+            const PairParam& p = MULTI ? ppl[ti * s.ntypes + (off[e] & 7u)] : p0;
+            if constexpr (MIXED)
+                lj_accum_mixed(p, X[e], Y[e], Z[e], R2[e], IN[e], acc);
+            else if constexpr (MULTI)
+                lj_accum(p, X[e], Y[e], Z[e], R2[e], IN[e], acc);
+            else
+                lj_accum_one(p, X[e], Y[e], Z[e], R2[e], IN[e], acc, nin);
+        }
     }
+    return acc;
 }
 
 // FP32 parameters of one type pair for the mixed pair loop with FP32 staging (32 bytes:
@@ -1443,103 +1734,83 @@ __device__ __forceinline__ PairF pair_f32(const PairParam& p)
     return PairF{p.r2f, p.sig2f, p.c4f, p.c24f, p.c48f, p.ucutf, p.r2s32, 0.0f};
 }
 
-// The mixed pair loop over one atom's list with FP32 tile-relative staging (SoA Px, Py, Pz
+// One list group of the mixed pair loop with FP32 tile-relative staging (SoA Px, Py, Pz
 // of SCAP + 1 floats, contiguous): displacement, r^2, cutoff and LJ arithmetic in FP32
-// (LennardJones::compute_potential, lennard_jones.rs:32-55, in FP32), the 8 entries of a
-// list group summed in FP32 and each group's sums added into the FP64 accumulators.
+// (LennardJones::compute_potential, lennard_jones.rs:32-55, in FP32), the 8 entries of the
+// group summed in FP32; sum_list adds each group's sums into the FP64 accumulators.
 // Entries are byte offsets of a float slot with the partner type in the two low bits; the
 // padding slot lies kPadFar away, so padding entries have r^2 = +inf and fail the cutoff.
 // A candidate outside the cutoff enters the reciprocal as +inf (v_rcp_f32 gives +0), so
 // its force factor and virial term are -0; the energy shift is masked.
 template <int SCAP, bool MULTI>
-__device__ __forceinline__ void atom_forces_f32(const SysDev& s, const float* Px, const PairF* prow,
-                                                const PairF& p0, int a, float qx, float qy, float qz,
-                                                Acc& acc)
+__device__ __forceinline__ Acc32 group_f32(const float* Px, const PairF* prow, const PairF& p0, u32x4 u, float qx,
+                                           float qy, float qz, uint32_t& nin)
 {
     constexpr uint32_t YO = (SCAP + 1) * 4, ZO = 2 * (SCAP + 1) * 4;
-    const int nn = gbl(s.nnb)[a];
-    const int ng = (nn + 7) >> 3;
-    const gu32x4* L = (const gu32x4*)(s.nbr + a);
     const char* bx = reinterpret_cast<const char*>(Px);
-    u32x4 un = {0u, 0u, 0u, 0u};
-    if (ng > 0) un = L[0];
-    uint32_t nin = 0;  // single species: pairs within the cutoff
-    for (int gi = 0; gi < ng; ++gi) {
-        const u32x4 u = un;
-        if (gi + 1 < ng) un = L[(size_t)(gi + 1) * s.npad];
-        const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
-        uint32_t off[8];
-        float X[8], Y[8], Z[8];
+    const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
+    uint32_t off[8];
+    float X[8], Y[8], Z[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        off[e] = (wv[e >> 1] >> ((e & 1) * 16)) & 0xffffu;
+        const uint32_t ad = MULTI ? off[e] & ~3u : off[e];
+        X[e] = *reinterpret_cast<const float*>(bx + ad);
+        Y[e] = *reinterpret_cast<const float*>(bx + ad + YO);
+        Z[e] = *reinterpret_cast<const float*>(bx + ad + ZO);
+    }
+    if constexpr (!MULTI) {
+        // one species, coordinates in sigma units: 1/r'^2 is (sigma/r)^2 itself; the
+        // energy and the pair virial follow from the sums of (sigma/r)^12 and (sigma/r)^6
+        // and the number of pairs in range (combined per atom after the loop), and the
+        // force sum is scaled back by 1/sigma there (finish_one_species)
+        float fx = 0.0f, fy = 0.0f, fz = 0.0f, s12 = 0.0f, s6 = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            off[e] = (wv[e >> 1] >> ((e & 1) * 16)) & 0xffffu;
-            const uint32_t ad = MULTI ? off[e] & ~3u : off[e];
-            X[e] = *reinterpret_cast<const float*>(bx + ad);
-            Y[e] = *reinterpret_cast<const float*>(bx + ad + YO);
-            Z[e] = *reinterpret_cast<const float*>(bx + ad + ZO);
-        }
-        if constexpr (!MULTI) {
-            // one species, coordinates in sigma units: 1/r'^2 is (sigma/r)^2 itself; the
-            // energy and the pair virial follow from the sums of (sigma/r)^12 and (sigma/r)^6
-            // and the number of pairs in range (combined per atom after the loop), and the
-            // force sum is scaled back by 1/sigma there
-            float fx = 0.0f, fy = 0.0f, fz = 0.0f, s12 = 0.0f, s6 = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float dx = X[e] - qx, dy = Y[e] - qy, dz = Z[e] - qz;
-                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                const float sr2 = __builtin_amdgcn_rcpf(cut_and_count(r2, p0.r2s, __builtin_inff(), nin));
-                const float sr6 = sr2 * sr2 * sr2;
-                const float fp = fmaf(p0.c48, sr6, -p0.c24) * sr6 * sr2;
-                fx = fmaf(-fp, dx, fx);
-                fy = fmaf(-fp, dy, fy);
-                fz = fmaf(-fp, dz, fz);
-                s12 = fmaf(sr6, sr6, s12);
-                s6 += sr6;
-            }
-            acc.fx += (double)fx;
-            acc.fy += (double)fy;
-            acc.fz += (double)fz;
-            acc.pe += (double)s12;
-            acc.wp += (double)s6;
-            continue;
-        }
-        float fx = 0.0f, fy = 0.0f, fz = 0.0f, pe = 0.0f, wp = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const PairF p = MULTI ? prow[off[e] & 3u] : p0;
             const float dx = X[e] - qx, dy = Y[e] - qy, dz = Z[e] - qz;
             const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const bool in = r2 <= p.r2;
-            const float inv = __builtin_amdgcn_rcpf(in ? r2 : __builtin_inff());
-            const float sr2 = p.sig2 * inv;
+            const float sr2 = __builtin_amdgcn_rcpf(cut_and_count(r2, p0.r2s, __builtin_inff(), nin));
             const float sr6 = sr2 * sr2 * sr2;
-            const float w = fmaf(p.c48, sr6, -p.c24) * sr6;  // r . F_ij: the pair virial term
-            const float fp = w * inv;
-            const float uc = in ? p.ucut : 0.0f;
-            const float uu = fmaf(fmaf(p.c4, sr6, -p.c4), sr6, -uc);
+            const float fp = fmaf(p0.c48, sr6, -p0.c24) * sr6 * sr2;
             fx = fmaf(-fp, dx, fx);
             fy = fmaf(-fp, dy, fy);
             fz = fmaf(-fp, dz, fz);
-            pe += uu;
-            wp += w;
+            s12 = fmaf(sr6, sr6, s12);
+            s6 += sr6;
         }
-        acc.fx += (double)fx;
-        acc.fy += (double)fy;
-        acc.fz += (double)fz;
-        acc.pe += (double)pe;
-        acc.wp += (double)wp;
+        return Acc32{fx, fy, fz, s12, s6};
     }
-    if constexpr (!MULTI) {
-        // U = 4 eps ((s/r)^12 - (s/r)^6) - U(rc) and r . F = 48 eps (s/r)^12 - 24 eps (s/r)^6
-        const PairParam& pp = s.pp[0];
-        const double s12 = acc.pe, s6 = acc.wp;
-        acc.pe = pp.c4 * (s12 - s6) - pp.ucut * (double)nin;
-        acc.wp = pp.c48 * s12 - pp.c24 * s6;
-        acc.fx *= pp.isig;
-        acc.fy *= pp.isig;
-        acc.fz *= pp.isig;
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f, pe = 0.0f, wp = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const PairF p = MULTI ? prow[off[e] & 3u] : p0;
+        const float dx = X[e] - qx, dy = Y[e] - qy, dz = Z[e] - qz;
+        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const bool in = r2 <= p.r2;
+        const float inv = __builtin_amdgcn_rcpf(in ? r2 : __builtin_inff());
+        const float sr2 = p.sig2 * inv;
+        const float sr6 = sr2 * sr2 * sr2;
+        const float w = fmaf(p.c48, sr6, -p.c24) * sr6;  // r . F_ij: the pair virial term
+        const float fp = w * inv;
+        const float uc = in ? p.ucut : 0.0f;
+        const float uu = fmaf(fmaf(p.c4, sr6, -p.c4), sr6, -uc);
+        fx = fmaf(-fp, dx, fx);
+        fy = fmaf(-fp, dy, fy);
+        fz = fmaf(-fp, dz, fz);
+        pe += uu;
+        wp += w;
     }
+    return Acc32{fx, fy, fz, pe, wp};
+}
+
+// Energy and pair virial of a single-species atom from the sums of (sigma/r)^12 and
+// (sigma/r)^6 and the number of pairs in range:
+// U = 4 eps ((s/r)^12 - (s/r)^6) - U(rc) and r . F = 48 eps (s/r)^12 - 24 eps (s/r)^6.
+__device__ __forceinline__ void finish_one_species(const PairParam& pp, uint32_t nin, Acc& acc)
+{
+    const double s12 = acc.pe, s6 = acc.wp;
+    acc.pe = pp.c4 * (s12 - s6) - pp.ucut * (double)nin;
+    acc.wp = pp.c48 * s12 - pp.c24 * s6;
 }
 
 // LDS of a force workgroup; T is the staged coordinate type.  The FP32 staging reads only
@@ -1575,29 +1846,121 @@ struct StageType<true> {
 #ifndef PIS_FORCE_MIN_WAVES_F32
 #define PIS_FORCE_MIN_WAVES_F32 4
 #endif
-template <bool MIXED, int KIND>
+template <bool MIXED, int KIND, int KL>
 struct ForceWaves {
     static constexpr bool F32 = MIXED && (KIND == KIND_ORTHO || KIND == KIND_TRI);
-    static constexpr int value = KIND == KIND_TRI_RAW ? 1
+    static constexpr int value = KIND == KIND_TRI_RAW            ? 1
+                                 : F32 && KIND == KIND_TRI && KL > 1 ? 3  // 4 would spill
                                  : F32                ? PIS_FORCE_MIN_WAVES_F32
                                  : MIXED              ? PIS_FORCE_MIN_WAVES_MIXED
                                                       : PIS_FORCE_MIN_WAVES_FP64;
 };
 
+// Pair sums of own atom a (position xi, yi, zi; nn list entries) by the KL lanes that share
+// it; un: the lane's first list group.
+template <int SCAP, bool MIXED, int KIND, int KL, class Lds>
+__device__ __forceinline__ Acc atom_sums(const SysDev& s, const State& st, const TileGeom& g, const Lds& lds,
+                                         double scale, double cx, double cy, double cz, int a, int ti, double xi,
+                                         double yi, double zi, int nn, u32x4 un)
+{
+    constexpr bool REL = KIND == KIND_ORTHO || KIND == KIND_TRI;
+    constexpr bool TRI = KIND == KIND_TRI || KIND == KIND_TRI_RAW;
+    constexpr bool F32 = MIXED && REL;
+    const int nt = s.ntypes, ng = (nn + 7) >> 3;
+    const gu32x4* L = (const gu32x4*)(s.nbr + a);
+    const PairParam p0 = s.pp[0];  // uniform: scalar loads, no vector registers
+    double qx = xi, qy = yi, qz = zi;
+    if (REL) rel_to_center(s, cx, cy, cz, qx, qy, qz);
+    Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if constexpr (F32) {
+        const PairF p0f = pair_f32(p0);
+        const float* Px = reinterpret_cast<const float*>(lds.Px);
+        uint32_t nin = 0;
+        if (nt == 1) {
+            const float fx = (float)(qx * scale), fy = (float)(qy * scale), fz = (float)(qz * scale);
+            sum_list<KL>(L, s.npad, ng, un, acc, nin, [&](int, u32x4 u, uint32_t& n) {
+                return group_f32<SCAP, false>(Px, lds.pf, p0f, u, fx, fy, fz, n);
+            });
+            finish_one_species(p0, nin, acc);
+            acc.fx *= p0.isig;  // from sigma units
+            acc.fy *= p0.isig;
+            acc.fz *= p0.isig;
+        } else {
+            const float fx = (float)qx, fy = (float)qy, fz = (float)qz;
+            sum_list<KL>(L, s.npad, ng, un, acc, nin, [&](int, u32x4 u, uint32_t& n) {
+                return group_f32<SCAP, true>(Px, lds.pf + ti * nt, p0f, u, fx, fy, fz, n);
+            });
+        }
+    } else {
+        const double* Px = reinterpret_cast<const double*>(lds.Px);
+        const double* Py = reinterpret_cast<const double*>(lds.Py);
+        const double* Pz = reinterpret_cast<const double*>(lds.Pz);
+        const ExactCtx ex = {&s, &st, lds.pref, lds.ecell, g.ne, xi, yi, zi};
+        uint32_t nin = 0;
+        if (nt == 1) {
+            sum_list<KL>(L, s.npad, ng, un, acc, nin, [&](int k, u32x4 u, uint32_t& n) {
+                return group_f64<SCAP, MIXED, false, !REL, TRI>(s, Px, Py, Pz, lds.ppl, p0, k, u, nn, ti, qx, qy, qz, ex, n);
+            });
+            if constexpr (!MIXED) finish_one_species(p0, nin, acc);
+        } else {
+            sum_list<KL>(L, s.npad, ng, un, acc, nin, [&](int k, u32x4 u, uint32_t& n) {
+                return group_f64<SCAP, MIXED, true, !REL, TRI>(s, Px, Py, Pz, lds.ppl, p0, k, u, nn, ti, qx, qy, qz, ex, n);
+            });
+        }
+    }
+    return acc;
+}
+
+// What a quad's lane needs of own atom a besides its neighbours: component min(sub, 2) of
+// position, velocity, force and build-time position, the type, the list length and the first
+// group of the lane's stream (requested before the length is known: the group is inside the
+// list's memory, and unused where the list is shorter).
+struct Own {
+    double x, v, f, r;
+    int type, nn;
+    u32x4 un;
+};
+
+__device__ __forceinline__ Own own_fetch(const SysDev& s, const State& st, int a, int sub, int integrate)
+{
+    const size_t at = (size_t)min(sub, 2) * s.npad + a;
+    Own o;
+    o.x = gbl(st.x)[at];
+    o.v = gbl(st.vx)[at];
+    o.f = integrate ? gbl(st.fx)[at] : 0.0;
+    o.r = integrate ? gbl(s.rx)[at] : 0.0;
+    o.type = gbl(st.type)[a];
+    o.nn = gbl(s.nnb)[a];
+    o.un = u32x4{0u, 0u, 0u, 0u};
+    if (sub < s.maxnb >> 3) o.un = ((const gu32x4*)(s.nbr + a))[(size_t)sub * s.npad];
+    return o;
+}
+
+__device__ __forceinline__ double pick3(int c, double x, double y, double z) { return c == 0 ? x : c == 1 ? y : z; }
+
 // KIND: one of KIND_ORTHO, KIND_TRI (tile-relative staging), KIND_ORTHO_RAW, KIND_TRI_RAW
 // (raw staging with a per-pair image).  Mixed precision with tile-relative staging stages
 // FP32 coordinates (atom_forces_f32); every other combination stages FP64.
-template <int SCAP, bool MIXED, int KIND>
-__global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND>::value)) void k_force(
+//
+// KL = 1: a workgroup per tile, a lane per atom.  KL = 4 (small launches, see class_lanes): four
+// workgroups per tile, each with 64 of every 256 of the tile's atoms and four lanes per atom.
+// A lone small system leaves most of the chip idle, and its time is one workgroup's chain of
+// latencies: this cuts the chain of list groups and spreads the pairs over four times the
+// CUs, for four times the staging.  Both give the same bits.
+template <int SCAP, bool MIXED, int KIND, int KL>
+__global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value)) void k_force(
     const SysDev* __restrict__ sys, const WorkItem* __restrict__ tiles, int ntw, int integrate)
 {
+    static_assert(KL == 1 || KL == 4, "one lane per atom or a quad");
+    __shared__ double mass[kMaxTypes];
     constexpr bool REL = KIND == KIND_ORTHO || KIND == KIND_TRI;
     constexpr bool TRI = KIND == KIND_TRI || KIND == KIND_TRI_RAW;
     constexpr bool F32 = MIXED && REL;
     typedef typename StageType<F32>::type T;
     __shared__ ForceLds<T, SCAP> lds;
 
-    const WorkItem w = tiles[xcd_remap(blockIdx.x, ntw)];
+    const int item = xcd_remap(blockIdx.x, ntw * KL), part = item % KL;
+    const WorkItem w = tiles[item / KL];
     const SysDev& s = sys[w.sys];
     if (system_kind(s) != KIND) return;             // another instantiation takes this tile
     if (integrate && s.ctl[CTL_LEFT] == 0) return;  // frozen system: the whole block leaves
@@ -1625,40 +1988,31 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND>::value)) voi
     }
     // the single-species FP32 loop works in sigma units (an absent pair keeps scale 1)
     const double scale = (F32 && nt == 1 && s.pp[0].r2_force >= 0.0) ? s.pp[0].isig : 1.0;
-    const int total = stage_tile<SCAP, REL ? STAGE_REL : STAGE_RAW, T>(
+    // four lanes per atom: the first atom's data and first list group are requested before the
+    // staging, whose latency they share
+    const int sub = (int)threadIdx.x % KL;
+    int a0 = 0, a1 = 0;
+    Own own = {};
+    if constexpr (KL > 1) {
+        if ((int)threadIdx.x < nt) mass[threadIdx.x] = s.mass[threadIdx.x];
+        own_atoms(s, g, w.idx, &a0, &a1);
+        a0 += part * 64 + (int)threadIdx.x / KL;
+        if (a0 < a1) own = own_fetch(s, st, a0, sub, integrate);
+    }
+    const int total = stage_tile<SCAP, REL ? STAGE_REL : STAGE_RAW, T, (KL > 1)>(
         s, st, g, cx, cy, cz, lds.Px, lds.Py, lds.Pz, (uint8_t*)nullptr, lds.pref, lds.ecell, lds.stmp,
-        ForceLds<T, SCAP>::MAP ? lds.smap : (uint8_t*)nullptr, scale);
+        KL == 1 && ForceLds<T, SCAP>::MAP ? lds.smap : (uint8_t*)nullptr, scale);
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
-    if (total <= SCAP) {
-        const PairParam p0 = s.pp[0];  // uniform: scalar loads, no vector registers
-        const PairF p0f = pair_f32(p0);
-        const int a0 = gbl(s.cell_start)[g.c0], a1 = gbl(s.cell_start)[g.c1];
-        for (int a = a0 + (int)threadIdx.x; a < a1; a += blockDim.x) {
+    if (total > SCAP) {
+        if (threadIdx.x == 0) atomicOr(&s.ctl[CTL_OVF_STAGE], 1);
+    } else if constexpr (KL == 1) {
+        own_atoms(s, g, w.idx, &a0, &a1);
+        for (int a = a0 + (int)threadIdx.x; a < a1; a += kTileThreads) {
             const double xi = gbl(st.x)[a], yi = gbl(st.y)[a], zi = gbl(st.z)[a];
-            const int ti = gbl(st.type)[a];
-            double qx = xi, qy = yi, qz = zi;
-            if (REL) rel_to_center(s, cx, cy, cz, qx, qy, qz);
-            Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
-            if constexpr (F32) {
-                const float* Px = reinterpret_cast<const float*>(lds.Px);
-                if (nt == 1)
-                    atom_forces_f32<SCAP, false>(s, Px, lds.pf, p0f, a, (float)(qx * scale), (float)(qy * scale),
-                                                 (float)(qz * scale), acc);
-                else
-                    atom_forces_f32<SCAP, true>(s, Px, lds.pf + ti * nt, p0f, a, (float)qx, (float)qy, (float)qz,
-                                                acc);
-            } else {
-                const double* Px = reinterpret_cast<const double*>(lds.Px);
-                const double* Py = reinterpret_cast<const double*>(lds.Py);
-                const double* Pz = reinterpret_cast<const double*>(lds.Pz);
-                const ExactCtx ex = {&s, &st, lds.pref, lds.ecell, g.ne, xi, yi, zi};
-                if (nt == 1)
-                    atom_forces<SCAP, MIXED, false, !REL, TRI>(s, Px, Py, Pz, lds.ppl, p0, a, ti, qx, qy, qz, ex,
-                                                               acc);
-                else
-                    atom_forces<SCAP, MIXED, true, !REL, TRI>(s, Px, Py, Pz, lds.ppl, p0, a, ti, qx, qy, qz, ex,
-                                                              acc);
-            }
+            const int ti = gbl(st.type)[a], nn = gbl(s.nnb)[a];
+            u32x4 un = {0u, 0u, 0u, 0u};
+            if (nn > 0) un = *(const gu32x4*)(s.nbr + a);
+            const Acc acc = atom_sums<SCAP, MIXED, KIND, KL>(s, st, g, lds, scale, cx, cy, cz, a, ti, xi, yi, zi, nn, un);
             const double m = s.mass[ti];
             // positions again from memory (L2): not held in registers across the pair loop
             const double xa = gbl(st.x)[a], ya = gbl(st.y)[a], za = gbl(st.z)[a];
@@ -1734,12 +2088,89 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND>::value)) voi
             sum[2] += (xa * acc.fx + ya * acc.fy) + za * acc.fz;
             sum[3] += acc.wp;
         }
-    } else if (threadIdx.x == 0) {
-        atomicOr(&s.ctl[CTL_OVF_STAGE], 1);
+    } else {
+        // Four lanes per atom: lane c < 3 of the quad finishes component c of the atom
+        // (everything it needs was requested before the staging), so the update's memory
+        // round trip and divisions are paid once, not per component.
+        for (int a = a0; a < a1; a += kTileThreads) {
+            const Own o = own;
+            if (a + kTileThreads < a1) own = own_fetch(s, st, a + kTileThreads, sub, integrate);
+            const double xi = quad_bcast<0>(o.x), yi = quad_bcast<1>(o.x), zi = quad_bcast<2>(o.x);
+            const Acc acc = atom_sums<SCAP, MIXED, KIND, KL>(s, st, g, lds, scale, cx, cy, cz, a, o.type, xi, yi, zi,
+                                                             o.nn, o.un);
+            const int c = min(sub, 2);
+            const size_t at = (size_t)c * s.npad + a;  // the x, y, z arrays of a vector lie npad apart
+            const double m = mass[o.type], f = pick3(c, acc.fx, acc.fy, acc.fz);
+            double v = o.v;
+            if (integrate) {
+                // the same operations as above, a component per lane
+                const double dt = s.dt;
+                v = v + ((o.f / m + f / m) * 0.5) * dt;
+                if (s.nhc_on) v = v * s.nhc[NHC_SCALE];
+                double x = o.x;
+                if (ahead) {
+                    x = x + (v * dt + (f / m) * 0.5 * s.dt2);
+                    double d2;
+                    if (TRI) {
+                        double X = quad_bcast<0>(x), Y = quad_bcast<1>(x), Z = quad_bcast<2>(x);
+                        wrap_tri(s.box, X, Y, Z);
+                        x = pick3(c, X, Y, Z);
+                        double ddx = X - quad_bcast<0>(o.r), ddy = Y - quad_bcast<1>(o.r), ddz = Z - quad_bcast<2>(o.r);
+                        mi_tri_fast(s.box, ddx, ddy, ddz);
+                        d2 = ddx * ddx + ddy * ddy + ddz * ddz;
+                    } else {
+                        const double L = pick3(c, s.L[0], s.L[1], s.L[2]);
+                        const double Li = pick3(c, s.Linv[0], s.Linv[1], s.Linv[2]);
+                        double sx = x * Li;
+                        sx = sx - floor(sx);
+                        x = L * sx;
+                        const double d = mi_fast(x - o.r, L, Li), q = d * d;
+                        d2 = quad_bcast<0>(q) + quad_bcast<1>(q) + quad_bcast<2>(q);
+                    }
+                    if (sub == 0 && !(d2 <= s.half_skin2)) {  // also catches NaN
+                        atomicOr(&s.ctl[CTL_REBUILD_NEXT], 1);
+                        if (d2 != d2) atomicOr(&s.ctl[CTL_NAN], 1);
+                    }
+                }
+                if (sub < 3) {
+                    gbl(wt.vx)[at] = v;
+                    gbl(wt.fx)[at] = f;
+                    gbl(wt.x)[at] = x;
+                } else if (rebuilt) {
+                    gbl(wt.type)[a] = (uint8_t)o.type;
+                    gbl(wt.orig)[a] = gbl(st.orig)[a];
+                }
+            } else if (sub < 3) {
+                gbl(st.fx)[at] = f;
+            }
+            const double vv = v * v, xf = o.x * f;
+            const double ke = 0.5 * m * ((quad_bcast<0>(vv) + quad_bcast<1>(vv)) + quad_bcast<2>(vv));
+            const double wa = (quad_bcast<0>(xf) + quad_bcast<1>(xf)) + quad_bcast<2>(xf);
+            sum[0] += acc.pe;  // the same in the quad's four lanes
+            sum[1] += ke;
+            sum[2] += wa;
+            sum[3] += acc.wp;
+        }
     }
-    block_sum4(sum, lds.rtmp);
+    double* P = s.partial + 4 * ((size_t)part * s.ntile + w.idx);
+    if constexpr (KL == 1) {
+        block_sum4(sum, lds.rtmp);
+    } else {
+        // this part's 64 atoms are the lanes of one wave of the KL = 1 kernel: a wave here holds
+        // one of its rows of 16, summed in the same order (wave_sum), then the four rows
+        for (int k = 0; k < 4; ++k) {
+            double v = sum[k];
+            v += dpp_f64<0x141>(v);  // row_half_mirror: the next quad
+            v += dpp_f64<0x140>(v);  // row_mirror: the next two
+            v = (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
+            if (threadIdx.x % 64 == 0) lds.rtmp[(threadIdx.x / 64) * 4 + k] = v;
+        }
+        __syncthreads();
+        for (int k = 0; k < 4; ++k)
+            sum[k] = (lds.rtmp[k] + lds.rtmp[4 + k]) + (lds.rtmp[8 + k] + lds.rtmp[12 + k]);
+    }
     if (threadIdx.x == 0) {
-        double* P = s.partial + 4 * (size_t)w.idx;
+        if (w.idx == 0 && part == 0) s.partial[16 * (size_t)s.ntile] = KL;
         P[0] = sum[0];
         P[1] = sum[1];
         P[2] = sum[2];
@@ -1778,9 +2209,18 @@ __device__ __forceinline__ void sum_partials(const SysDev& s, double* v, double*
 {
     v[0] = v[1] = v[2] = v[3] = 0.0;
     const __attribute__((address_space(1))) double* P = gbl(static_cast<const double*>(s.partial));
-    // four tiles' partials in flight per thread (the loop is latency-bound otherwise)
     const int bd = blockDim.x;
     int t = threadIdx.x;
+    if (P[16 * s.ntile] > 1.0) {  // parts of the launch that wrote them
+        // four parts per tile, added as block_sum4 adds a tile's four waves
+        for (; t < s.ntile; t += bd)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const __attribute__((address_space(1))) double* p = P + 4 * t + k;
+                v[k] += ((p[0] + p[4 * s.ntile]) + p[8 * s.ntile]) + p[12 * s.ntile];
+            }
+    }
+    // four tiles' partials in flight per thread (the loop is latency-bound otherwise)
     for (; t + 3 * bd < s.ntile; t += 4 * bd) {
         double q[4][4];
 #pragma unroll
@@ -2316,7 +2756,8 @@ __global__ __launch_bounds__(kTileThreads) void k_list_to_orig(const SysDev* __r
                                                     nullptr, pref, ecell, stmp);
     if (total > SCAP) return;
     const int* Li = reinterpret_cast<const int*>(Px);
-    const int a0 = s.cell_start[g.c0], a1 = s.cell_start[g.c1];
+    int a0, a1;
+    own_atoms(s, g, w.idx, &a0, &a1);
     for (int a = a0 + (int)threadIdx.x; a < a1; a += blockDim.x) {
         const uint32_t oa = st.orig[a];
         const int nn = s.nnb[a];
@@ -2359,7 +2800,8 @@ __global__ __launch_bounds__(kTileThreads) void k_list_digest(const SysDev* __re
     const int total = stage_tile<SCAP, STAGE_INDEX, int>(s, st, g, 0.0, 0.0, 0.0, Li, nullptr, nullptr, nullptr,
                                                          pref, ecell, stmp);
     if (total > SCAP) return;
-    const int a0 = s.cell_start[g.c0], a1 = s.cell_start[g.c1];
+    int a0, a1;
+    own_atoms(s, g, w.idx, &a0, &a1);
     for (int a = a0 + (int)threadIdx.x; a < a1; a += blockDim.x) {
         const int nn = s.nnb[a];
         uint64_t h = 0;
@@ -2454,12 +2896,19 @@ void launch_rebuild_sort(hipStream_t st, const SysDev* d_sys, int nsys, const Wo
 }
 
 void launch_build_list(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work, int n_tile_work,
-                       int scap, int kinds)
+                       int scap, int kinds, int lanes)
 {
     if (n_tile_work <= 0) return;
-    const int gt = grid_cap(n_tile_work, PIS_BUILD_GRID_CAP);
+    const int gt = grid_cap(n_tile_work * lanes, PIS_BUILD_GRID_CAP);
+#define PIS_BUILD_KL(S, K, KL) \
+    hipLaunchKernelGGL((k_build_list<S, K, KL>), dim3(gt), dim3(kTileThreads), 0, st, d_sys, tile_work, n_tile_work)
 #define PIS_BUILD_K(S, K) \
-    hipLaunchKernelGGL((k_build_list<S, K>), dim3(gt), dim3(kTileThreads), 0, st, d_sys, tile_work, n_tile_work)
+    do { \
+        if (lanes == 1) \
+            PIS_BUILD_KL(S, K, 1); \
+        else \
+            PIS_BUILD_KL(S, K, 4); \
+    } while (0)
 #define PIS_BUILD_O(S) PIS_BUILD_K(S, KIND_ORTHO)
 #define PIS_BUILD_OR(S) PIS_BUILD_K(S, KIND_ORTHO_RAW)
 #define PIS_BUILD_T(S) PIS_BUILD_K(S, KIND_TRI)
@@ -2469,6 +2918,7 @@ void launch_build_list(hipStream_t st, const SysDev* d_sys, const WorkItem* tile
     if (kinds & KIND_TRI) PIS_SCAP_DISPATCH(scap, PIS_BUILD_T);
     if (kinds & KIND_TRI_RAW) PIS_SCAP_DISPATCH(scap, PIS_BUILD_TR);
 #undef PIS_BUILD_K
+#undef PIS_BUILD_KL
 #undef PIS_BUILD_O
 #undef PIS_BUILD_OR
 #undef PIS_BUILD_T
@@ -2476,20 +2926,27 @@ void launch_build_list(hipStream_t st, const SysDev* d_sys, const WorkItem* tile
 }
 
 void launch_force(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work, int n_tile_work,
-                  int scap, bool mixed, int integrate, int kinds)
+                  int scap, bool mixed, int integrate, int kinds, int lanes)
 {
     if (n_tile_work <= 0) return;
-    const dim3 g(n_tile_work), b(kTileThreads);
-#define PIS_FORCE_LAUNCH(S, M, K) \
-    hipLaunchKernelGGL((k_force<S, M, K>), g, b, 0, st, d_sys, tile_work, n_tile_work, integrate)
-#define PIS_FORCE_M(S) PIS_FORCE_LAUNCH(S, true, KIND_ORTHO)
-#define PIS_FORCE_D(S) PIS_FORCE_LAUNCH(S, false, KIND_ORTHO)
-#define PIS_FORCE_MT(S) PIS_FORCE_LAUNCH(S, true, KIND_TRI)
-#define PIS_FORCE_DT(S) PIS_FORCE_LAUNCH(S, false, KIND_TRI)
-#define PIS_FORCE_MR(S) PIS_FORCE_LAUNCH(S, true, KIND_TRI_RAW)
-#define PIS_FORCE_DR(S) PIS_FORCE_LAUNCH(S, false, KIND_TRI_RAW)
-#define PIS_FORCE_MO(S) PIS_FORCE_LAUNCH(S, true, KIND_ORTHO_RAW)
-#define PIS_FORCE_DO(S) PIS_FORCE_LAUNCH(S, false, KIND_ORTHO_RAW)
+    const dim3 g(n_tile_work * lanes), b(kTileThreads);
+#define PIS_FORCE_LAUNCH(S, M, K, KL) \
+    hipLaunchKernelGGL((k_force<S, M, K, KL>), g, b, 0, st, d_sys, tile_work, n_tile_work, integrate)
+#define PIS_FORCE_PICK(S, M, K) \
+    do { \
+        if (lanes == 1) \
+            PIS_FORCE_LAUNCH(S, M, K, 1); \
+        else \
+            PIS_FORCE_LAUNCH(S, M, K, 4); \
+    } while (0)
+#define PIS_FORCE_M(S) PIS_FORCE_PICK(S, true, KIND_ORTHO)
+#define PIS_FORCE_D(S) PIS_FORCE_PICK(S, false, KIND_ORTHO)
+#define PIS_FORCE_MT(S) PIS_FORCE_PICK(S, true, KIND_TRI)
+#define PIS_FORCE_DT(S) PIS_FORCE_PICK(S, false, KIND_TRI)
+#define PIS_FORCE_MR(S) PIS_FORCE_PICK(S, true, KIND_TRI_RAW)
+#define PIS_FORCE_DR(S) PIS_FORCE_PICK(S, false, KIND_TRI_RAW)
+#define PIS_FORCE_MO(S) PIS_FORCE_PICK(S, true, KIND_ORTHO_RAW)
+#define PIS_FORCE_DO(S) PIS_FORCE_PICK(S, false, KIND_ORTHO_RAW)
     if (kinds & KIND_ORTHO) {
         if (mixed)
             PIS_SCAP_DISPATCH(scap, PIS_FORCE_M);
@@ -2515,6 +2972,7 @@ void launch_force(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work
             PIS_SCAP_DISPATCH(scap, PIS_FORCE_DR);
     }
 #undef PIS_FORCE_LAUNCH
+#undef PIS_FORCE_PICK
 #undef PIS_FORCE_M
 #undef PIS_FORCE_D
 #undef PIS_FORCE_MT

@@ -57,10 +57,6 @@ __global__ __launch_bounds__(256) void k_noalloc_setup(const NoAllocSetup a)
         const int x = i % d.nc[0], y = (i / d.nc[0]) % d.nc[1], z = i / (d.nc[0] * d.nc[1]);
         d.nat2sorted[i] = sorted_cell_id(d.nc, d.tile, x, y, z);
     }
-    for (int t = gid; t <= d.ntile; t += stride)
-        d.tile_cell0[t] = t < d.ntile ? tile_first_cell(d.nc, d.tile, t % d.nt[0], (t / d.nt[0]) % d.nt[1],
-                                                        t / (d.nt[0] * d.nt[1]))
-                                      : d.ncell;
     for (int k = gid; k < a.n_atom_work; k += stride) a.atom_work[k] = WorkItem{0, k * kAtomThreads};
     for (int k = gid; k < a.n_tile_work; k += stride) a.tile_work[k] = WorkItem{0, k};
     for (int k = gid; k < d.ntypes * d.ntypes; k += stride) const_cast<PairParam*>(d.pp)[k] = a.pp[k];
@@ -164,6 +160,7 @@ extern "C" pis_status pis_compute_potential_noalloc(const pis_system_desc* desc,
     carve_system(p, Lo, b, a.dev);
     a.dev.thermo = (ThermoDev*)(b + o_th);
     a.dev.thermo_cap = 1;
+    const int lanes = class_lanes(p.ntile);
     a.dev_slot = (SysDev*)(b + o_sys);
     a.atom_work = (WorkItem*)(b + o_aw);
     a.tile_work = (WorkItem*)(b + o_tw);
@@ -176,7 +173,7 @@ extern "C" pis_status pis_compute_potential_noalloc(const pis_system_desc* desc,
     const size_t n16 = off / 16;
     hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)std::min<size_t>((n16 + 255) / 256, 2048)), dim3(256), 0, st,
                        (uint4*)base, n16);
-    const int work = std::max(std::max(p.ncell, p.ntile + 1), std::max(n_aw, p.ntile));
+    const int work = std::max(p.ncell, std::max(n_aw, p.ntile));
     hipLaunchKernelGGL(k_noalloc_setup, dim3((unsigned)std::min((work + 255) / 256, 1024)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(k_load_typed, dim3((unsigned)n_aw), dim3(kAtomThreads), 0, st, d_sys, d_pos, d_types);
     // the list at these positions, as pis_set_state builds it: sort, build, flip, labels;
@@ -185,7 +182,7 @@ extern "C" pis_status pis_compute_potential_noalloc(const pis_system_desc* desc,
     int32_t ctl[CTL_COUNT];
     for (int pass = 0; pass < 2; ++pass) {
         launch_rebuild_sort(st, d_sys, 1, a.atom_work, n_aw);
-        launch_build_list(st, d_sys, a.tile_work, p.ntile, p.scap, kind);
+        launch_build_list(st, d_sys, a.tile_work, p.ntile, p.scap, kind, lanes);
         launch_flip(st, d_sys, 1);
         launch_sync_labels(st, d_sys, a.atom_work, n_aw);
         PIS_HIP(hipGetLastError());
@@ -210,7 +207,7 @@ extern "C" pis_status pis_compute_potential_noalloc(const pis_system_desc* desc,
     if (ctl[CTL_OVF_NB])
         return fail(PIS_ERR_CAPACITY, "neighbour capacity " + std::to_string(p.maxnb) + " exceeded (" +
                                           std::to_string(ctl[CTL_MAXNB]) + " needed)");
-    launch_force(st, d_sys, a.tile_work, p.ntile, p.scap, p.mixed, 0, kind);
+    launch_force(st, d_sys, a.tile_work, p.ntile, p.scap, p.mixed, 0, kind, lanes);
     launch_reduce(st, d_sys, 1, 1, 1, 0);
     hipLaunchKernelGGL(k_store_forces_add, dim3((unsigned)std::max(n_aw, 1)), dim3(kAtomThreads), 0, st, d_sys,
                        d_forces_inout, d_pe);
