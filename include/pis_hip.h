@@ -193,8 +193,9 @@ pis_status pis_get_neighbor_list(pis_ctx* ctx, uint64_t* offsets, uint32_t* idx,
 pis_status pis_get_list_digest(pis_ctx* ctx, uint32_t* counts, uint64_t* hashes);
 
 pis_status pis_get_stats(pis_ctx* ctx, pis_stats* out);
-/* Replay one captured hipGraph per step in pis_verlet_step_nve / pis_batch_verlet_step_nve
- * (1) instead of launching each kernel (0, the default).  Ignored while kernel timing is on. */
+/* Replay one captured hipGraph per step of a batch (1) instead of launching each kernel (0,
+ * the default).  Ignored while kernel timing is on, and by contexts of one system: their
+ * steps are launched kernel by kernel either way, the list's rebuild only when it is due. */
 pis_status pis_set_graph_mode(pis_ctx* ctx, int32_t enable);
 /* Turn per-launch HIP-event timing of the force kernel on (1) or off (0); resets sums. */
 pis_status pis_set_kernel_timing(pis_ctx* ctx, int32_t enable);

@@ -40,7 +40,8 @@ enum {
     CTL_REBUILD_NEXT = 11,  // skin check of those advanced positions
     CTL_BOX = 12,      // the box (NPT) became too thin for the planned cell grid
     CTL_BADINPUT = 13, // device-resident input rejected: bit 0 atom type, bit 1 position
-    CTL_COUNT = 14
+    CTL_DONE = 14,     // steps completed in the current call
+    CTL_COUNT = 15
 };
 
 // Device-resident box of a system (SysDev::box): h and h^-1 column-major, |det h|.  The
@@ -147,6 +148,9 @@ struct SysDev {
     double cellw[3];
     double half_skin2;     // (skin/2)^2
     double wslack;         // x-window slack of the list build: FP32 staging error + margin
+    // host-visible progress of a host-driven run (steps completed << 1 | a rebuild is due), null
+    // otherwise
+    unsigned long long* progress;
     double dt, dt2;
     double kb, volume;
     int32_t n, npad, ntypes, maxnb;
@@ -164,6 +168,15 @@ struct SysDev {
     int32_t nblk;          // 256-atom blocks (npad / 256, rounded up)
     int32_t list_shift;    // list entry = (LDS slot << list_shift) | partner type: 3 when the
                            // force kernel stages FP64 coordinates (8-byte slots), 2 for FP32
+};
+
+// Gate of a host-driven step (launches of a single system's run, see drive_steps): `step` is
+// the index of the step the launch belongs to, or -1 for launches that always run.  A
+// launch whose predecessors are not all done, or whose list is due, does nothing; `fresh`
+// marks the force and reduction behind the launches that rebuild the list.
+struct StepGate {
+    int32_t step;
+    int32_t fresh;
 };
 
 // Cell numbering.  Cells are numbered tile-major: tiles in x-fastest order, and inside a

@@ -140,6 +140,8 @@ struct pis_ctx {
     double* d_snap = nullptr;
     size_t snap_bytes = 0;
     bool snap_pending = false;
+    // host-driven runs of a single system: the progress word its steps write (pinned)
+    unsigned long long* progress = nullptr;
     // statistics / timing
     uint64_t steps = 0, force_launches = 0;
     bool timing = false;
@@ -163,7 +165,7 @@ pis_status reserve_lanes(pis_ctx* c, int nlanes);
 pis_status ensure_xfer(pis_ctx* c, size_t bytes);
 pis_status read_ctl(pis_ctx* c, uint32_t k, int32_t* ctl);
 pis_status write_ctl(pis_ctx* c, uint32_t k, const int32_t* ctl);
-pis_status enqueue_classes(pis_ctx* c, bool build, int force);
+pis_status enqueue_classes(pis_ctx* c, bool build, int force, StepGate gate = StepGate{-1, 0});
 // KIND_* bits of the context's systems (which build/force instantiations a launch needs)
 inline int plan_kind(const Plan& p)
 {

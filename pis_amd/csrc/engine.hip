@@ -484,6 +484,7 @@ void pis::carve_system(const Plan& p, const Layout& Lo, char* b, SysDev& d)
     d.mass = (const double*)(b + Lo.m);
     d.nhc = (double*)(b + Lo.nhc);
     d.nhc_on = 0;
+    d.progress = nullptr;
     d.box = (double*)(b + Lo.box);
     d.npt = (double*)(b + Lo.npt);
     d.tens = (double*)(b + Lo.tens);
@@ -606,6 +607,7 @@ void pis::free_ctx(pis_ctx* c)
     if (c->d_atom_work) (void)hipFree(c->d_atom_work);
     if (c->d_tile_work) (void)hipFree(c->d_tile_work);
     if (c->d_xfer) (void)hipFree(c->d_xfer);
+    if (c->progress) (void)hipHostFree(c->progress);
     if (c->snap_stream) {
         (void)hipStreamSynchronize(c->snap_stream);
         (void)hipStreamDestroy(c->snap_stream);
@@ -873,7 +875,7 @@ pis_status pis::write_ctl(pis_ctx* c, uint32_t k, const int32_t* ctl)
 // lane l > 0 run on side[l-1], forked after everything already on `stream` and joined
 // before anything enqueued later; captured into a graph, the fork becomes parallel
 // branches.
-pis_status pis::enqueue_classes(pis_ctx* c, bool build, int force)
+pis_status pis::enqueue_classes(pis_ctx* c, bool build, int force, StepGate gate)
 {
     const int nl = c->nlanes;
     if (nl > 1) {
@@ -883,7 +885,7 @@ pis_status pis::enqueue_classes(pis_ctx* c, bool build, int force)
     for (const auto& q : c->classes) {
         hipStream_t st = q.lane == 0 ? c->stream : c->side[q.lane - 1];
         if (build) launch_build_list(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, q.kind, q.lanes);
-        if (force >= 0) launch_force(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, c->mixed, force, q.kind, q.lanes);
+        if (force >= 0) launch_force(st, c->d_sys, c->d_tile_work + q.first, q.count, q.scap, c->mixed, force, q.kind, q.lanes, gate);
     }
     for (int l = 1; l < nl; ++l) {
         PIS_HIP(hipEventRecord(c->join[l - 1], c->side[l - 1]));
@@ -1121,7 +1123,7 @@ static pis_status batch_compute(pis_ctx* c, pis_thermo* out /* [nsys] or null */
     PIS_TRY(run_rebuild(c));
     launch_set_ctl(c->stream, c->d_sys, (int)c->sys.size(), CTL_STEP, 0);
     PIS_TRY(launch_force_timed(c, 0));
-    launch_reduce(c->stream, c->d_sys, (int)c->sys.size(), 1, 1, 0);
+    launch_reduce(c->stream, c->d_sys, (int)c->sys.size(), 1, 1, 0, StepGate{-1, 0});
     PIS_HIP(hipGetLastError());
     PIS_HIP(hipStreamSynchronize(c->stream));
     PIS_TRY(collect_timing(c));
@@ -1142,7 +1144,7 @@ static pis_status enqueue_one(pis_ctx* c, bool first, bool record, bool nvt, boo
 {
     const int ns = (int)c->sys.size();
     if (nvt && (first || npt)) launch_nhc_pre(c->stream, c->d_sys, ns);
-    if (first || nvt) launch_integrate_pos(c->stream, c->d_sys, c->d_atom_work, c->n_atom_work);
+    if (first || nvt) launch_integrate_pos(c->stream, c->d_sys, c->d_atom_work, c->n_atom_work, StepGate{-1, 0});
     launch_rebuild_sort(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work);
     if (timed) {
         // timed: every list build first, then the force launches between events
@@ -1152,7 +1154,7 @@ static pis_status enqueue_one(pis_ctx* c, bool first, bool record, bool nvt, boo
         PIS_TRY(enqueue_classes(c, true, 1));
         c->force_launches++;
     }
-    launch_reduce(c->stream, c->d_sys, ns, 1, record ? 1 : 0, 1);
+    launch_reduce(c->stream, c->d_sys, ns, 1, record ? 1 : 0, 1, StepGate{-1, 0});
     return PIS_OK;
 }
 
@@ -1194,6 +1196,57 @@ pis_status pis::enqueue_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
             if ((t & 255) == 0) PIS_HIP(hipGetLastError());
         }
     }
+    return PIS_OK;
+}
+
+// nsteps of NVE (or NVT) of a context's only system, driven by the host: a step is its force
+// and reduction (and NVT's position update), and the five list-rebuild kernels are launched
+// only when a step reports that the skin check fired, instead of in every step of a fixed
+// sequence (they cost 17 us of a 240 us step at 1M atoms even when they return at once, and
+// half of the step at 4000).  The step's progress arrives in a word of pinned memory; up to
+// `ahead` steps are queued beyond the last one known to be done, and those queued behind a
+// due rebuild find themselves gated off (StepGate) and are queued again behind it.
+static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt)
+{
+    constexpr uint64_t ahead = 3;
+    volatile unsigned long long* word = c->progress;
+    *word = 0;
+    auto step = [&](uint64_t k, bool position, bool fresh) -> pis_status {
+        const StepGate gate{(int32_t)k, fresh ? 1 : 0};
+        if (position) launch_integrate_pos(c->stream, c->d_sys, c->d_atom_work, c->n_atom_work, gate);
+        if (fresh) launch_rebuild_sort(c->stream, c->d_sys, 1, c->d_atom_work, c->n_atom_work);
+        PIS_TRY(enqueue_classes(c, fresh, 1, gate));
+        launch_reduce(c->stream, c->d_sys, 1, 1, record ? 1 : 0, 1, gate);
+        return PIS_OK;
+    };
+    if (nvt) launch_nhc_pre(c->stream, c->d_sys, 1);
+    PIS_TRY(step(0, true, true));
+    uint64_t queued = 1, done = 0, listed = 0;  // listed: the last step queued with a rebuild
+    for (unsigned idle = 0; done < nsteps;) {
+        while (queued < nsteps && queued < done + ahead) PIS_TRY(step(queued++, nvt, false));
+        const unsigned long long now = *word;
+        if ((now >> 1) > done) idle = 0;
+        done = now >> 1;
+        if ((now & 1) && done < nsteps && listed < done) {
+            // step `done` waits for a new list, and what is queued behind it does nothing
+            PIS_TRY(step(done, false, true));
+            listed = done;
+            queued = done + 1;
+            idle = 0;
+        } else if (++idle == 1u << 16) {
+            // nothing for milliseconds: a stream that has run dry will not move any more
+            idle = 0;
+            PIS_HIP(hipGetLastError());
+            const hipError_t e = hipStreamQuery(c->stream);
+            (void)hipGetLastError();  // "not ready" is no error of this run
+            if (e != hipErrorNotReady && *word == now && !((now & 1) && listed < done)) {
+                if (e != hipSuccess) return fail(PIS_ERR_HIP, std::string("run: ") + hipGetErrorString(e));
+                return fail(PIS_ERR_HIP, "the run stopped after " + std::to_string(done) + " steps");
+            }
+        }
+        __builtin_ia32_pause();
+    }
+    c->force_launches += nsteps;
     return PIS_OK;
 }
 
@@ -1277,6 +1330,13 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
     // downloaded before the next starts.
     // NPT runs in chunks of kNptChunk steps: a system whose box would become thinner than
     // its cell grid freezes on the device, and the host re-plans it between chunks.
+    const bool driven = c->sys.size() == 1 && !npt && !c->timing;
+    if (driven && !c->progress) {
+        void* p = nullptr;
+        PIS_HIP(hipHostMalloc(&p, 64, hipHostMallocDefault));
+        c->progress = (unsigned long long*)p;
+    }
+    for (auto& h : c->sys) h.dev.progress = driven ? c->progress : nullptr;
     constexpr uint64_t kThermoFloor = 1024, kThermoChunk = 8192, kNptChunk = 64;
     uint64_t chunk = out ? std::min(nsteps, kThermoChunk) : nsteps;
     if (npt) chunk = std::min(chunk, kNptChunk);
@@ -1292,8 +1352,7 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
     bool resumed = false;  // the chunk starts on a re-planned system
     for (uint64_t done = 0; done < nsteps;) {
         const uint64_t k = std::min(chunk, nsteps - done);
-        launch_set_ctl(c->stream, c->d_sys, ns, CTL_LEFT, -1);
-        launch_set_ctl(c->stream, c->d_sys, ns, CTL_STEP, 0);
+        launch_begin_run(c->stream, c->d_sys, ns, (int)std::min<uint64_t>(k, (uint64_t)INT32_MAX));
         if (npt) {
             // verlet_step_npt_mtk (potential.rs:112-135): barostat and box update, the NVT
             // step on the scaled state, the second scaling and momentum update; direct
@@ -1309,6 +1368,8 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
                 launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 2, rec);
                 if ((t & 63) == 0) PIS_HIP(hipGetLastError());
             }
+        } else if (driven) {
+            PIS_TRY(drive_steps(c, k, out != nullptr, nvt));
         } else {
             PIS_TRY(enqueue_steps(c, k, out != nullptr, nvt));
         }

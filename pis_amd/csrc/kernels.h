@@ -11,7 +11,7 @@ void launch_store_aos(hipStream_t st, const SysDev* d_sys, int sys, int n, doubl
 void launch_set_ctl(hipStream_t st, const SysDev* d_sys, int nsys, int slot, int value);
 
 void launch_integrate_pos(hipStream_t st, const SysDev* d_sys, const WorkItem* atom_work,
-                          int n_atom_work);
+                          int n_atom_work, StepGate gate);
 // Counting sort of every system whose rebuild flag is set (bin, scan, scatter, rank).
 void launch_rebuild_sort(hipStream_t st, const SysDev* d_sys, int nsys, const WorkItem* atom_work,
                          int n_atom_work);
@@ -20,10 +20,12 @@ void launch_rebuild_sort(hipStream_t st, const SysDev* d_sys, int nsys, const Wo
 void launch_build_list(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work, int n_tile_work,
                        int scap, int kinds, int lanes);
 void launch_force(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work,
-                  int n_tile_work, int scap, bool mixed, int integrate, int kinds, int lanes);
+                  int n_tile_work, int scap, bool mixed, int integrate, int kinds, int lanes, StepGate gate);
 // `step` = 1 after an NVE step: frozen systems (ctl[CTL_LEFT] == 0) are skipped and a
 // positive step budget is counted down.
-void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int record, int step);
+void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int record, int step, StepGate gate);
+// Control words of a run of `remain` steps: no frozen systems, first record, no step done.
+void launch_begin_run(hipStream_t st, const SysDev* d_sys, int nsys, int remain);
 void launch_gather_ctl(hipStream_t st, const SysDev* d_sys, int nsys, int32_t* out);
 // NVT: start-of-step chain update and velocity scale; reset of the run's step counter.
 void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys);

@@ -550,6 +550,20 @@ __device__ __forceinline__ int search_sorted(const float* P, int lo, int hi, dou
 // ---------------------------------------------------------------------------------
 // state transfer
 
+// Whether a gated launch of a run does its step (StepGate).
+__device__ __forceinline__ bool step_runs(const StepGate& gate, int done, int rebuild)
+{
+    return gate.step < 0 || (done == gate.step && (gate.fresh || !rebuild));
+}
+
+// The run's progress for the host that drives it: one 8-byte store, nothing else is read by it.
+__device__ __forceinline__ void tell_progress(const SysDev& s, int done, bool due)
+{
+    if (s.progress)
+        __hip_atomic_store(s.progress, ((unsigned long long)done << 1) | (due ? 1ull : 0ull), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void k_load_aos(const SysDev* __restrict__ sys, int k, const double* __restrict__ pos,
                            const double* __restrict__ vel, const double* __restrict__ force,
                            const uint8_t* __restrict__ type)
@@ -596,6 +610,17 @@ __global__ void k_store_aos(const SysDev* __restrict__ sys, int k, double* __res
     }
 }
 
+__global__ void k_begin_run(const SysDev* __restrict__ sys, int nsys, int remain)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nsys) return;
+    int32_t* ctl = sys[k].ctl;
+    ctl[CTL_LEFT] = -1;
+    ctl[CTL_STEP] = 0;
+    ctl[CTL_REMAIN] = remain;
+    ctl[CTL_DONE] = 0;
+}
+
 __global__ void k_set_ctl(const SysDev* __restrict__ sys, int nsys, int slot, int value)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -606,13 +631,14 @@ __global__ void k_set_ctl(const SysDev* __restrict__ sys, int nsys, int slot, in
 // integrator, first half (potential.rs:16-22) + skin trigger
 
 __global__ __launch_bounds__(kAtomThreads) void k_integrate_pos(const SysDev* __restrict__ sys,
-                                                                 const WorkItem* __restrict__ work)
+                                                                 const WorkItem* __restrict__ work, StepGate gate)
 {
     const WorkItem w = work[blockIdx.x];
     const SysDev& s = sys[w.sys];
     const int a = w.idx + threadIdx.x;
-    if (a >= s.n || s.ctl[CTL_LEFT] == 0) return;
-    const State st = s.st[__builtin_amdgcn_readfirstlane(s.ctl[CTL_CUR])];
+    const int left = gbl(s.ctl)[CTL_LEFT], done = gbl(s.ctl)[CTL_DONE], cur = gbl(s.ctl)[CTL_CUR];
+    if (a >= s.n || left == 0 || (gate.step >= 0 && done != gate.step)) return;
+    const State st = s.st[__builtin_amdgcn_readfirstlane(cur)];
     const double m = gbl(s.mass)[gbl(st.type)[a]];
     const double dt = s.dt, dt2 = s.dt2;
     double vx = gbl(st.vx)[a], vy = gbl(st.vy)[a], vz = gbl(st.vz)[a];
@@ -1860,20 +1886,18 @@ struct ForceWaves {
 // it; un: the lane's first list group.
 template <int SCAP, bool MIXED, int KIND, int KL, class Lds>
 __device__ __forceinline__ Acc atom_sums(const SysDev& s, const State& st, const TileGeom& g, const Lds& lds,
-                                         double scale, double cx, double cy, double cz, int a, int ti, double xi,
-                                         double yi, double zi, int nn, u32x4 un)
+                                         const PairParam& p0, const PairF& p0f, double scale, double cx, double cy,
+                                         double cz, int a, int ti, double xi, double yi, double zi, int nn, u32x4 un)
 {
     constexpr bool REL = KIND == KIND_ORTHO || KIND == KIND_TRI;
     constexpr bool TRI = KIND == KIND_TRI || KIND == KIND_TRI_RAW;
     constexpr bool F32 = MIXED && REL;
     const int nt = s.ntypes, ng = (nn + 7) >> 3;
     const gu32x4* L = (const gu32x4*)(s.nbr + a);
-    const PairParam p0 = s.pp[0];  // uniform: scalar loads, no vector registers
     double qx = xi, qy = yi, qz = zi;
     if (REL) rel_to_center(s, cx, cy, cz, qx, qy, qz);
     Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
     if constexpr (F32) {
-        const PairF p0f = pair_f32(p0);
         const float* Px = reinterpret_cast<const float*>(lds.Px);
         uint32_t nin = 0;
         if (nt == 1) {
@@ -1949,7 +1973,7 @@ __device__ __forceinline__ double pick3(int c, double x, double y, double z) { r
 // CUs, for four times the staging.  Both give the same bits.
 template <int SCAP, bool MIXED, int KIND, int KL>
 __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value)) void k_force(
-    const SysDev* __restrict__ sys, const WorkItem* __restrict__ tiles, int ntw, int integrate)
+    const SysDev* __restrict__ sys, const WorkItem* __restrict__ tiles, int ntw, int integrate, StepGate gate)
 {
     static_assert(KL == 1 || KL == 4, "one lane per atom or a quad");
     __shared__ double mass[kMaxTypes];
@@ -1963,21 +1987,30 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
     const WorkItem w = tiles[item / KL];
     const SysDev& s = sys[w.sys];
     if (system_kind(s) != KIND) return;             // another instantiation takes this tile
-    if (integrate && s.ctl[CTL_LEFT] == 0) return;  // frozen system: the whole block leaves
+    // control words: all requested at once (one round trip)
+    const __attribute__((address_space(1))) int32_t* ctl = gbl(static_cast<const int32_t*>(s.ctl));
+    const int c_cur = ctl[CTL_CUR], c_rb = ctl[CTL_REBUILD], c_left = ctl[CTL_LEFT];
+    const int c_remain = ctl[CTL_REMAIN], c_done = ctl[CTL_DONE];
+    if (integrate && c_left == 0) return;  // frozen system: the whole block leaves
+    if (!step_runs(gate, c_done, c_rb)) {
+        // the host learns of a list that is due (NVT's position update found it) here
+        if (blockIdx.x == 0 && threadIdx.x == 0 && c_done == gate.step) tell_progress(s, c_done, true);
+        return;
+    }
     // read set: the live set, or the freshly sorted one on a rebuild step; a step writes
     // its results into the other set (wt), which becomes live at the end of the step
     // (control words are read with vector loads; readfirstlane makes the block-uniform
     // choices scalar, so the state pointers stay in scalar registers)
-    const int cur = __builtin_amdgcn_readfirstlane(s.ctl[CTL_CUR]);
-    const int rbf = __builtin_amdgcn_readfirstlane(s.ctl[CTL_REBUILD]);
+    const int cur = __builtin_amdgcn_readfirstlane(c_cur);
+    const int rbf = __builtin_amdgcn_readfirstlane(c_rb);
     const int rset = cur ^ (rbf ? 1 : 0);
     const State st = s.st[rset];
     const State wt = s.st[rset ^ 1];
     const bool rebuilt = rbf != 0;
     // while more steps of this call follow (and no thermostat must act in between), the
     // next step's position update happens here, from the v and F just computed
-    const bool ahead = integrate && __builtin_amdgcn_readfirstlane(s.ctl[CTL_REMAIN]) > 1 &&
-                       __builtin_amdgcn_readfirstlane(s.ctl[CTL_LEFT]) != 1 && !s.nhc_on;
+    const bool ahead = integrate && __builtin_amdgcn_readfirstlane(c_remain) > 1 &&
+                       __builtin_amdgcn_readfirstlane(c_left) != 1 && !s.nhc_on;
     const TileGeom g = tile_geom(s, w.idx);
     double cx, cy, cz;
     tile_center(s, g, cx, cy, cz);
@@ -2002,6 +2035,10 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
     const int total = stage_tile<SCAP, REL ? STAGE_REL : STAGE_RAW, T, (KL > 1)>(
         s, st, g, cx, cy, cz, lds.Px, lds.Py, lds.Pz, (uint8_t*)nullptr, lds.pref, lds.ecell, lds.stmp,
         KL == 1 && ForceLds<T, SCAP>::MAP ? lds.smap : (uint8_t*)nullptr, scale);
+    // read once, ahead of the atoms' stores: uniform, so scalar registers (read per atom they
+    // would be vector loads whose wait in the pair loop also waits for the list's prefetch)
+    const PairParam p0 = s.pp[0];
+    const PairF p0f = pair_f32(p0);
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
     if (total > SCAP) {
         if (threadIdx.x == 0) atomicOr(&s.ctl[CTL_OVF_STAGE], 1);
@@ -2012,7 +2049,8 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
             const int ti = gbl(st.type)[a], nn = gbl(s.nnb)[a];
             u32x4 un = {0u, 0u, 0u, 0u};
             if (nn > 0) un = *(const gu32x4*)(s.nbr + a);
-            const Acc acc = atom_sums<SCAP, MIXED, KIND, KL>(s, st, g, lds, scale, cx, cy, cz, a, ti, xi, yi, zi, nn, un);
+            const Acc acc = atom_sums<SCAP, MIXED, KIND, KL>(s, st, g, lds, p0, p0f, scale, cx, cy, cz, a, ti, xi, yi,
+                                                             zi, nn, un);
             const double m = s.mass[ti];
             // positions again from memory (L2): not held in registers across the pair loop
             const double xa = gbl(st.x)[a], ya = gbl(st.y)[a], za = gbl(st.z)[a];
@@ -2096,8 +2134,8 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
             const Own o = own;
             if (a + kTileThreads < a1) own = own_fetch(s, st, a + kTileThreads, sub, integrate);
             const double xi = quad_bcast<0>(o.x), yi = quad_bcast<1>(o.x), zi = quad_bcast<2>(o.x);
-            const Acc acc = atom_sums<SCAP, MIXED, KIND, KL>(s, st, g, lds, scale, cx, cy, cz, a, o.type, xi, yi, zi,
-                                                             o.nn, o.un);
+            const Acc acc = atom_sums<SCAP, MIXED, KIND, KL>(s, st, g, lds, p0, p0f, scale, cx, cy, cz, a, o.type, xi,
+                                                             yi, zi, o.nn, o.un);
             const int c = min(sub, 2);
             const size_t at = (size_t)c * s.npad + a;  // the x, y, z arrays of a vector lie npad apart
             const double m = mass[o.type], f = pick3(c, acc.fx, acc.fy, acc.fz);
@@ -2635,7 +2673,7 @@ __device__ void note_list_box(const SysDev& s)
 }
 
 __global__ __launch_bounds__(1024) void k_reduce(const SysDev* __restrict__ sys, int flip, int record,
-                                                 int step)
+                                                 int step, StepGate gate)
 {
     __shared__ double rtmp[64];
     const SysDev& s = sys[blockIdx.x];
@@ -2644,10 +2682,11 @@ __global__ __launch_bounds__(1024) void k_reduce(const SysDev* __restrict__ sys,
     __attribute__((address_space(1))) int32_t* ctl = gbl(s.ctl);
     const int c_cur = ctl[CTL_CUR], c_rb = ctl[CTL_REBUILD], c_nrb = ctl[CTL_NREBUILD];
     const int c_step = ctl[CTL_STEP], c_next = ctl[CTL_REBUILD_NEXT];
-    const int c_remain = ctl[CTL_REMAIN], c_left = ctl[CTL_LEFT];
+    const int c_remain = ctl[CTL_REMAIN], c_left = ctl[CTL_LEFT], c_done = ctl[CTL_DONE];
     double v[4];
     sum_partials(s, v, rtmp);
-    if (step && c_left == 0) return;  // frozen: no step was taken (uniform over the block)
+    // frozen, or a gated step that did not run: no step was taken (uniform over the block)
+    if (step && (c_left == 0 || !step_runs(gate, c_done, c_rb))) return;
     if (threadIdx.x != 0) return;
     const double pe = 0.5 * v[0], ke = v[1], wabs = v[2], wpair = 0.5 * v[3];
     double ham = pe + ke;
@@ -2695,6 +2734,8 @@ __global__ __launch_bounds__(1024) void k_reduce(const SysDev* __restrict__ sys,
         ctl[CTL_REBUILD_NEXT] = 0;
         if (c_remain > 0) ctl[CTL_REMAIN] = c_remain - 1;
         if (c_left > 0) ctl[CTL_LEFT] = c_left - 1;
+        ctl[CTL_DONE] = c_done + 1;
+        tell_progress(s, c_done + 1, c_next != 0);
     } else if (flip && c_rb) {
         ctl[CTL_CUR] = c_cur ^ 1;
         ctl[CTL_REBUILD] = 0;
@@ -2877,9 +2918,9 @@ void launch_set_ctl(hipStream_t st, const SysDev* d_sys, int nsys, int slot, int
 }
 
 void launch_integrate_pos(hipStream_t st, const SysDev* d_sys, const WorkItem* atom_work,
-                          int n_atom_work)
+                          int n_atom_work, StepGate gate)
 {
-    hipLaunchKernelGGL(k_integrate_pos, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work);
+    hipLaunchKernelGGL(k_integrate_pos, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, gate);
 }
 
 void launch_rebuild_sort(hipStream_t st, const SysDev* d_sys, int nsys, const WorkItem* atom_work,
@@ -2926,12 +2967,12 @@ void launch_build_list(hipStream_t st, const SysDev* d_sys, const WorkItem* tile
 }
 
 void launch_force(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work, int n_tile_work,
-                  int scap, bool mixed, int integrate, int kinds, int lanes)
+                  int scap, bool mixed, int integrate, int kinds, int lanes, StepGate gate)
 {
     if (n_tile_work <= 0) return;
     const dim3 g(n_tile_work * lanes), b(kTileThreads);
 #define PIS_FORCE_LAUNCH(S, M, K, KL) \
-    hipLaunchKernelGGL((k_force<S, M, K, KL>), g, b, 0, st, d_sys, tile_work, n_tile_work, integrate)
+    hipLaunchKernelGGL((k_force<S, M, K, KL>), g, b, 0, st, d_sys, tile_work, n_tile_work, integrate, gate)
 #define PIS_FORCE_PICK(S, M, K) \
     do { \
         if (lanes == 1) \
@@ -2983,9 +3024,14 @@ void launch_force(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work
 #undef PIS_FORCE_DO
 }
 
-void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int record, int step)
+void launch_begin_run(hipStream_t st, const SysDev* d_sys, int nsys, int remain)
 {
-    hipLaunchKernelGGL(k_reduce, dim3(nsys), dim3(1024), 0, st, d_sys, flip, record, step);
+    hipLaunchKernelGGL(k_begin_run, dim3((nsys + 255) / 256), dim3(256), 0, st, d_sys, nsys, remain);
+}
+
+void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int record, int step, StepGate gate)
+{
+    hipLaunchKernelGGL(k_reduce, dim3(nsys), dim3(1024), 0, st, d_sys, flip, record, step, gate);
 }
 
 void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys)

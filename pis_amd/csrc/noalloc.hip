@@ -207,8 +207,8 @@ extern "C" pis_status pis_compute_potential_noalloc(const pis_system_desc* desc,
     if (ctl[CTL_OVF_NB])
         return fail(PIS_ERR_CAPACITY, "neighbour capacity " + std::to_string(p.maxnb) + " exceeded (" +
                                           std::to_string(ctl[CTL_MAXNB]) + " needed)");
-    launch_force(st, d_sys, a.tile_work, p.ntile, p.scap, p.mixed, 0, kind, lanes);
-    launch_reduce(st, d_sys, 1, 1, 1, 0);
+    launch_force(st, d_sys, a.tile_work, p.ntile, p.scap, p.mixed, 0, kind, lanes, StepGate{-1, 0});
+    launch_reduce(st, d_sys, 1, 1, 1, 0, StepGate{-1, 0});
     hipLaunchKernelGGL(k_store_forces_add, dim3((unsigned)std::max(n_aw, 1)), dim3(kAtomThreads), 0, st, d_sys,
                        d_forces_inout, d_pe);
     PIS_HIP(hipGetLastError());
