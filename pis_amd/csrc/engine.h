@@ -133,6 +133,10 @@ struct pis_ctx {
     int max_lanes = pis::kMaxLanes;  // streams the classes may spread over (the first is `stream`)
     void* d_xfer = nullptr;
     size_t xfer_bytes = 0;
+    void* h_pin = nullptr;  // pinned staging of small transfers (at most kPinnedMax bytes)
+    size_t pin_bytes = 0;
+    std::vector<SysDev> sent;  // descriptors as last uploaded to d_sys
+    bool listed = false;  // the only system's list is known to be current (no rebuild pending)
     // trajectory snapshots: positions copied on `stream`, sent to the host on snap_stream
     // (default priority) while later steps run; one in flight at a time
     hipStream_t snap_stream = nullptr;
@@ -163,6 +167,9 @@ pis_status group_tiles(pis_ctx* c);
 // Side streams and events for `nlanes` lanes (created once, kept until the context ends).
 pis_status reserve_lanes(pis_ctx* c, int nlanes);
 pis_status ensure_xfer(pis_ctx* c, size_t bytes);
+// Pinned staging memory of at least `bytes` (at most kPinnedMax).
+constexpr size_t kPinnedMax = (size_t)4 << 20;
+pis_status ensure_pin(pis_ctx* c, size_t bytes);
 pis_status read_ctl(pis_ctx* c, uint32_t k, int32_t* ctl);
 pis_status write_ctl(pis_ctx* c, uint32_t k, const int32_t* ctl);
 pis_status enqueue_classes(pis_ctx* c, bool build, int force, StepGate gate = StepGate{-1, 0});

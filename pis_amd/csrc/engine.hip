@@ -589,8 +589,11 @@ pis_status pis::upload_sys(pis_ctx* c)
 {
     std::vector<SysDev> v(c->sys.size());
     for (size_t k = 0; k < c->sys.size(); ++k) v[k] = c->sys[k].dev;
+    if (v.size() == c->sent.size() && memcmp(v.data(), c->sent.data(), v.size() * sizeof(SysDev)) == 0) return PIS_OK;
+    c->sent.clear();
     PIS_HIP(hipMemcpyAsync(c->d_sys, v.data(), v.size() * sizeof(SysDev), hipMemcpyHostToDevice, c->stream));
     PIS_HIP(hipStreamSynchronize(c->stream));
+    c->sent = std::move(v);
     return PIS_OK;
 }
 
@@ -607,6 +610,7 @@ void pis::free_ctx(pis_ctx* c)
     if (c->d_atom_work) (void)hipFree(c->d_atom_work);
     if (c->d_tile_work) (void)hipFree(c->d_tile_work);
     if (c->d_xfer) (void)hipFree(c->d_xfer);
+    if (c->h_pin) (void)hipHostFree(c->h_pin);
     if (c->progress) (void)hipHostFree(c->progress);
     if (c->snap_stream) {
         (void)hipStreamSynchronize(c->snap_stream);
@@ -724,6 +728,7 @@ static pis_status relayout(pis_ctx* c)
     if (c->sys_cap < c->sys.size()) {
         if (c->d_sys) PIS_HIP(hipFree(c->d_sys));
         c->d_sys = nullptr;
+        c->sent.clear();
         const size_t cap = std::max<size_t>(c->sys.size(), 2 * c->sys_cap);
         PIS_HIP(hipMalloc(&c->d_sys, sizeof(SysDev) * cap));
         c->sys_cap = cap;
@@ -856,10 +861,25 @@ pis_status pis::ensure_xfer(pis_ctx* c, size_t bytes)
     return PIS_OK;
 }
 
+pis_status pis::ensure_pin(pis_ctx* c, size_t bytes)
+{
+    if (c->pin_bytes >= bytes) return PIS_OK;
+    const size_t grow = std::min(std::max({bytes, 2 * c->pin_bytes, (size_t)64 << 10}), kPinnedMax);
+    if (grow < bytes) return fail(PIS_ERR_INVALID_ARGUMENT, "transfer above the pinned staging limit");
+    if (c->h_pin) PIS_HIP(hipHostFree(c->h_pin));
+    c->h_pin = nullptr;
+    c->pin_bytes = 0;
+    PIS_HIP(hipHostMalloc(&c->h_pin, grow, hipHostMallocDefault));
+    c->pin_bytes = grow;
+    return PIS_OK;
+}
+
 pis_status pis::read_ctl(pis_ctx* c, uint32_t k, int32_t* ctl)
 {
-    PIS_HIP(hipMemcpyAsync(ctl, c->sys[k].dev.ctl, CTL_COUNT * 4, hipMemcpyDeviceToHost, c->stream));
+    PIS_TRY(ensure_pin(c, CTL_COUNT * 4));
+    PIS_HIP(hipMemcpyAsync(c->h_pin, c->sys[k].dev.ctl, CTL_COUNT * 4, hipMemcpyDeviceToHost, c->stream));
     PIS_HIP(hipStreamSynchronize(c->stream));
+    memcpy(ctl, c->h_pin, CTL_COUNT * 4);
     return PIS_OK;
 }
 
@@ -911,24 +931,67 @@ pis_status pis::run_rebuild(pis_ctx* c)
     return PIS_OK;
 }
 
+// Status of system k from its control words.
+static pis_status check_ctl(pis_ctx* c, uint32_t k, const int32_t* ctl)
+{
+    if (ctl[CTL_OVF_STAGE])
+        return fail(PIS_ERR_CAPACITY, "system " + std::to_string(k) + ": LDS staging capacity exceeded");
+    if (ctl[CTL_BOX])
+        return fail(PIS_ERR_CAPACITY, "system " + std::to_string(k) +
+                                          ": the box deformed below the planned cell grid (rcut + skin)");
+    if (ctl[CTL_OVF_NB])
+        return fail(PIS_ERR_CAPACITY, "system " + std::to_string(k) + ": neighbour capacity " +
+                                          std::to_string(c->sys[k].plan.maxnb) + " exceeded (" +
+                                          std::to_string(ctl[CTL_MAXNB]) + " needed)");
+    if (ctl[CTL_NAN])
+        return fail(PIS_ERR_NAN_ENERGY, "system " + std::to_string(k) + ": non-finite energy or position");
+    return PIS_OK;
+}
+
+// After everything queued on the stream: the control words of every system [nsys][CTL_COUNT]
+// and, if `out`, nrec thermo records per system [nrec][nsys] into `out`, with one wait.  The
+// records stay in c->h_pin (out untouched) until the caller has looked at the flags; more than
+// fit there are left for read_thermo (*pinned false).
+static pis_status collect_run(pis_ctx* c, uint64_t nrec, std::vector<int32_t>& ctl, bool* pinned)
+{
+    const size_t ns = c->sys.size(), nc = ns * CTL_COUNT * 4, nt = nrec * ns * sizeof(ThermoDev);
+    const size_t off = align256(nc);
+    *pinned = nrec > 0 && off + nt <= kPinnedMax;
+    ctl.resize(ns * CTL_COUNT);
+    if (off > kPinnedMax) {  // tens of thousands of systems
+        for (uint32_t k = 0; k < ns; ++k) PIS_TRY(read_ctl(c, k, &ctl[(size_t)k * CTL_COUNT]));
+        return PIS_OK;
+    }
+    const size_t bytes = *pinned ? off + nt : nc;
+    PIS_TRY(ensure_pin(c, bytes));
+    if (ns == 1) {
+        PIS_HIP(hipMemcpyAsync(c->h_pin, c->sys[0].dev.ctl, nc, hipMemcpyDeviceToHost, c->stream));
+        if (*pinned)
+            PIS_HIP(hipMemcpyAsync((char*)c->h_pin + off, c->sys[0].thermo, nt, hipMemcpyDeviceToHost, c->stream));
+    } else {
+        PIS_TRY(ensure_xfer(c, bytes));
+        launch_gather_ctl(c->stream, c->d_sys, (int)ns, (int32_t*)c->d_xfer);
+        if (*pinned)
+            launch_gather_thermo(c->stream, c->d_sys, (int)ns, (int)nrec, (ThermoDev*)((char*)c->d_xfer + off));
+        PIS_HIP(hipGetLastError());
+        PIS_HIP(hipMemcpyAsync(c->h_pin, c->d_xfer, bytes, hipMemcpyDeviceToHost, c->stream));
+    }
+    PIS_HIP(hipStreamSynchronize(c->stream));
+    memcpy(ctl.data(), c->h_pin, nc);
+    return PIS_OK;
+}
+
 pis_status pis::check_flags(pis_ctx* c, int only)
 {
-    for (uint32_t k = 0; k < c->sys.size(); ++k) {
-        if (only >= 0 && (int)k != only) continue;
+    if (only >= 0) {
         int32_t ctl[CTL_COUNT];
-        PIS_TRY(read_ctl(c, k, ctl));
-        if (ctl[CTL_OVF_STAGE])
-            return fail(PIS_ERR_CAPACITY, "system " + std::to_string(k) + ": LDS staging capacity exceeded");
-        if (ctl[CTL_BOX])
-            return fail(PIS_ERR_CAPACITY, "system " + std::to_string(k) +
-                                              ": the box deformed below the planned cell grid (rcut + skin)");
-        if (ctl[CTL_OVF_NB])
-            return fail(PIS_ERR_CAPACITY, "system " + std::to_string(k) + ": neighbour capacity " +
-                                              std::to_string(c->sys[k].plan.maxnb) + " exceeded (" +
-                                              std::to_string(ctl[CTL_MAXNB]) + " needed)");
-        if (ctl[CTL_NAN])
-            return fail(PIS_ERR_NAN_ENERGY, "system " + std::to_string(k) + ": non-finite energy or position");
+        PIS_TRY(read_ctl(c, (uint32_t)only, ctl));
+        return check_ctl(c, (uint32_t)only, ctl);
     }
+    std::vector<int32_t> ctl;
+    bool pinned;
+    PIS_TRY(collect_run(c, 0, ctl, &pinned));
+    for (uint32_t k = 0; k < c->sys.size(); ++k) PIS_TRY(check_ctl(c, k, &ctl[(size_t)k * CTL_COUNT]));
     return PIS_OK;
 }
 
@@ -983,17 +1046,27 @@ pis_status pis::sys_set_state(pis_ctx* c, uint32_t k, const double* pos, const d
     double* dv = dp + 3 * n;
     double* df = dv + 3 * n;
     uint8_t* dt = (uint8_t*)(df + 3 * n);
-    PIS_HIP(hipMemcpyAsync(dp, pos, 3 * n * 8, hipMemcpyHostToDevice, c->stream));
-    if (vel) PIS_HIP(hipMemcpyAsync(dv, vel, 3 * n * 8, hipMemcpyHostToDevice, c->stream));
-    if (force) PIS_HIP(hipMemcpyAsync(df, force, 3 * n * 8, hipMemcpyHostToDevice, c->stream));
-    PIS_HIP(hipMemcpyAsync(dt, h.plan.type0.data(), n, hipMemcpyHostToDevice, c->stream));
-    int32_t ctl[CTL_COUNT] = {0};
-    ctl[CTL_CUR] = 0;
-    ctl[CTL_REBUILD] = 1;
-    PIS_TRY(write_ctl(c, k, ctl));
+    const size_t v3 = 3 * n * 8, all = 3 * v3 + n;
+    c->listed = false;
+    if (all <= kPinnedMax) {
+        // one transfer from pinned memory: each of four from the caller's pageable memory waits
+        // for its own staging
+        PIS_TRY(ensure_pin(c, all));
+        char* p = (char*)c->h_pin;
+        memcpy(p, pos, v3);
+        if (vel) memcpy(p + v3, vel, v3);
+        if (force) memcpy(p + 2 * v3, force, v3);
+        memcpy(p + 3 * v3, h.plan.type0.data(), n);
+        PIS_HIP(hipMemcpyAsync(dp, p, all, hipMemcpyHostToDevice, c->stream));
+    } else {
+        PIS_HIP(hipMemcpyAsync(dp, pos, v3, hipMemcpyHostToDevice, c->stream));
+        if (vel) PIS_HIP(hipMemcpyAsync(dv, vel, v3, hipMemcpyHostToDevice, c->stream));
+        if (force) PIS_HIP(hipMemcpyAsync(df, force, v3, hipMemcpyHostToDevice, c->stream));
+        PIS_HIP(hipMemcpyAsync(dt, h.plan.type0.data(), n, hipMemcpyHostToDevice, c->stream));
+    }
+    int32_t ctl[CTL_COUNT];
     launch_load_aos(c->stream, c->d_sys, (int)k, (int)n, dp, vel ? dv : nullptr, force ? df : nullptr, dt);
     PIS_TRY(run_rebuild(c));
-    PIS_HIP(hipStreamSynchronize(c->stream));
     // The planned staging capacity assumes a uniform density.  A configuration with denser
     // spots (a lattice whose planes sit on cell faces, a cluster) that fills a tile's halo
     // to within 2 % + 16 atoms of the class gets a larger class, sized from the halo count
@@ -1019,9 +1092,11 @@ pis_status pis::sys_set_state(pis_ctx* c, uint32_t k, const double* pos, const d
         again[CTL_REBUILD] = 1;
         PIS_TRY(write_ctl(c, k, again));
         PIS_TRY(run_rebuild(c));
-        PIS_HIP(hipStreamSynchronize(c->stream));
+        PIS_TRY(read_ctl(c, k, ctl));
     }
-    return check_flags(c, (int)k);
+    PIS_TRY(check_ctl(c, k, ctl));
+    c->listed = c->sys.size() == 1;
+    return PIS_OK;
 }
 
 pis_status pis::sys_get_state(pis_ctx* c, uint32_t k, double* pos, double* vel, double* force)
@@ -1033,6 +1108,24 @@ pis_status pis::sys_get_state(pis_ctx* c, uint32_t k, double* pos, double* vel, 
     double* dp = (double*)c->d_xfer;
     double* dv = dp + 3 * n;
     double* df = dv + 3 * n;
+    const size_t v3 = 3 * n * 8;
+    double* want[3] = {pos, vel, force};
+    const size_t count = (pos ? 1 : 0) + (vel ? 1 : 0) + (force ? 1 : 0);
+    if (count && count * v3 <= kPinnedMax) {
+        // the wanted arrays side by side, one transfer into pinned memory
+        PIS_TRY(ensure_pin(c, count * v3));
+        double* at[3] = {nullptr, nullptr, nullptr};
+        size_t q = 0;
+        for (int j = 0; j < 3; ++j)
+            if (want[j]) at[j] = dp + 3 * n * q++;
+        launch_store_aos(c->stream, c->d_sys, (int)k, (int)n, at[0], at[1], at[2]);
+        PIS_HIP(hipGetLastError());
+        PIS_HIP(hipMemcpyAsync(c->h_pin, dp, count * v3, hipMemcpyDeviceToHost, c->stream));
+        PIS_HIP(hipStreamSynchronize(c->stream));
+        for (int j = 0; j < 3; ++j)
+            if (want[j]) memcpy(want[j], (char*)c->h_pin + ((char*)at[j] - (char*)dp), v3);
+        return PIS_OK;
+    }
     launch_store_aos(c->stream, c->d_sys, (int)k, (int)n, dp, dv, df);
     PIS_HIP(hipGetLastError());
     if (pos) PIS_HIP(hipMemcpyAsync(pos, dp, 3 * n * 8, hipMemcpyDeviceToHost, c->stream));
@@ -1092,6 +1185,8 @@ static pis_status collect_timing(pis_ctx* c)
     return PIS_OK;
 }
 
+static_assert(sizeof(ThermoDev) == sizeof(pis_thermo), "records are copied as they are");
+
 static pis_status read_thermo(pis_ctx* c, uint64_t nrec, pis_thermo* out)
 {
     const size_t ns = c->sys.size();
@@ -1120,18 +1215,21 @@ static pis_status batch_compute(pis_ctx* c, pis_thermo* out /* [nsys] or null */
     PIS_TRY(ensure_thermo(c, 1));
     // a pending rebuild (the last step's skin check fired, or the staging changed) first:
     // the list must hold every pair within the cutoff at these positions
-    PIS_TRY(run_rebuild(c));
+    if (!c->listed) PIS_TRY(run_rebuild(c));
     launch_set_ctl(c->stream, c->d_sys, (int)c->sys.size(), CTL_STEP, 0);
     PIS_TRY(launch_force_timed(c, 0));
     launch_reduce(c->stream, c->d_sys, (int)c->sys.size(), 1, 1, 0, StepGate{-1, 0});
     PIS_HIP(hipGetLastError());
+    std::vector<int32_t> ctl;
+    bool pinned;
+    PIS_TRY(collect_run(c, 1, ctl, &pinned));
     PIS_HIP(hipStreamSynchronize(c->stream));
     PIS_TRY(collect_timing(c));
-    PIS_TRY(check_flags(c));
-    std::vector<pis_thermo> t(c->sys.size());
-    PIS_TRY(read_thermo(c, 1, t.data()));
-    if (out)
-        for (size_t k = 0; k < t.size(); ++k) out[k] = t[k];
+    const size_t ns = c->sys.size();
+    for (uint32_t k = 0; k < ns; ++k) PIS_TRY(check_ctl(c, k, &ctl[(size_t)k * CTL_COUNT]));
+    if (!out) return PIS_OK;
+    if (!pinned) return read_thermo(c, 1, out);
+    memcpy(out, (char*)c->h_pin + align256(ns * CTL_COUNT * 4), ns * sizeof(pis_thermo));
     return PIS_OK;
 }
 
@@ -1220,17 +1318,18 @@ static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
         return PIS_OK;
     };
     if (nvt) launch_nhc_pre(c->stream, c->d_sys, 1);
-    PIS_TRY(step(0, true, true));
-    uint64_t queued = 1, done = 0, listed = 0;  // listed: the last step queued with a rebuild
+    PIS_TRY(step(0, true, false));
+    uint64_t queued = 1, done = 0;
+    int64_t listed = -1;  // the last step queued with a rebuild
     for (unsigned idle = 0; done < nsteps;) {
         while (queued < nsteps && queued < done + ahead) PIS_TRY(step(queued++, nvt, false));
         const unsigned long long now = *word;
         if ((now >> 1) > done) idle = 0;
         done = now >> 1;
-        if ((now & 1) && done < nsteps && listed < done) {
+        if ((now & 1) && done < nsteps && listed < (int64_t)done) {
             // step `done` waits for a new list, and what is queued behind it does nothing
             PIS_TRY(step(done, false, true));
-            listed = done;
+            listed = (int64_t)done;
             queued = done + 1;
             idle = 0;
         } else if (++idle == 1u << 16) {
@@ -1239,7 +1338,7 @@ static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
             PIS_HIP(hipGetLastError());
             const hipError_t e = hipStreamQuery(c->stream);
             (void)hipGetLastError();  // "not ready" is no error of this run
-            if (e != hipErrorNotReady && *word == now && !((now & 1) && listed < done)) {
+            if (e != hipErrorNotReady && *word == now && !((now & 1) && listed < (int64_t)done)) {
                 if (e != hipSuccess) return fail(PIS_ERR_HIP, std::string("run: ") + hipGetErrorString(e));
                 return fail(PIS_ERR_HIP, "the run stopped after " + std::to_string(done) + " steps");
             }
@@ -1330,6 +1429,7 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
     // downloaded before the next starts.
     // NPT runs in chunks of kNptChunk steps: a system whose box would become thinner than
     // its cell grid freezes on the device, and the host re-plans it between chunks.
+    c->listed = false;
     const bool driven = c->sys.size() == 1 && !npt && !c->timing;
     if (driven && !c->progress) {
         void* p = nullptr;
@@ -1374,11 +1474,11 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
             PIS_TRY(enqueue_steps(c, k, out != nullptr, nvt));
         }
         PIS_HIP(hipGetLastError());
-        PIS_HIP(hipStreamSynchronize(c->stream));
+        std::vector<int32_t> ctl;
+        bool pinned;
+        PIS_TRY(collect_run(c, out ? k : 0, ctl, &pinned));
         PIS_TRY(collect_timing(c));
         if (npt) {
-            int32_t ctl[CTL_COUNT];
-            PIS_TRY(read_ctl(c, 0, ctl));
             if (ns == 1 && ctl[CTL_BOX]) {
                 // the steps before the freeze are done; the one that froze is run again
                 double chain[NHC_COUNT];
@@ -1396,8 +1496,12 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
             }
         }
         c->steps += k;
-        PIS_TRY(check_flags(c));
-        if (out) PIS_TRY(read_thermo(c, k, out + done * (uint64_t)ns));
+        for (int q = 0; q < ns; ++q) PIS_TRY(check_ctl(c, (uint32_t)q, &ctl[(size_t)q * CTL_COUNT]));
+        if (out && pinned)
+            memcpy(out + done * (uint64_t)ns, (char*)c->h_pin + align256((size_t)ns * CTL_COUNT * 4),
+                   k * (size_t)ns * sizeof(pis_thermo));
+        else if (out)
+            PIS_TRY(read_thermo(c, k, out + done * (uint64_t)ns));
         done += k;
         resumed = false;
     }
@@ -1448,6 +1552,7 @@ static pis_status npt_init(pis_ctx* c, const pis_nhc_params* chain, const pis_mt
         return fail(PIS_ERR_INVALID_ARGUMENT, "pis_mtk_params.reserved must be 0");
     PIS_TRY(nvt_init(c, chain));
     bool relist = false;
+    c->listed = false;
     for (auto& h : c->sys) {
         // the box becomes general with the first step: raw staging with the general-box
         // image, bands for positions up to 1.25x the current extent (the box may grow)

@@ -4,6 +4,7 @@
 
 namespace pis {
 
+// State of system `sys` into buffer set 0, its control words reset and a rebuild requested.
 void launch_load_aos(hipStream_t st, const SysDev* d_sys, int sys, int n, const double* pos,
                      const double* vel, const double* force, const uint8_t* type);
 void launch_store_aos(hipStream_t st, const SysDev* d_sys, int sys, int n, double* pos,
@@ -27,6 +28,8 @@ void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int 
 // Control words of a run of `remain` steps: no frozen systems, first record, no step done.
 void launch_begin_run(hipStream_t st, const SysDev* d_sys, int nsys, int remain);
 void launch_gather_ctl(hipStream_t st, const SysDev* d_sys, int nsys, int32_t* out);
+// Thermo records of every system, [nrec][nsys].
+void launch_gather_thermo(hipStream_t st, const SysDev* d_sys, int nsys, int nrec, ThermoDev* out);
 // NVT: start-of-step chain update and velocity scale; reset of the run's step counter.
 void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys);
 void launch_nhc_run(hipStream_t st, const SysDev* d_sys, int nsys, uint64_t step0, uint64_t total);

@@ -570,6 +570,7 @@ __global__ void k_load_aos(const SysDev* __restrict__ sys, int k, const double* 
 {
     const SysDev& s = sys[k];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < CTL_COUNT) s.ctl[i] = i == CTL_REBUILD ? 1 : 0;
     if (i >= s.n) return;
     const State st = s.st[0];
     st.x[i] = pos[3 * i];
@@ -2751,6 +2752,13 @@ __global__ void k_gather_ctl(const SysDev* __restrict__ sys, int nsys, int32_t* 
     out[i] = sys[i / CTL_COUNT].ctl[i % CTL_COUNT];
 }
 
+// Thermo records [nrec][nsys] of every system, in one array.
+__global__ void k_gather_thermo(const SysDev* __restrict__ sys, int nsys, int nrec, ThermoDev* __restrict__ out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nsys * nrec) out[i] = sys[i % nsys].thermo[i / nsys];
+}
+
 // After a host-requested sort the set the next step writes into still holds the previous
 // order's types and original indices: copy them from the live set.
 __global__ __launch_bounds__(kAtomThreads) void k_sync_labels(const SysDev* __restrict__ sys,
@@ -3049,6 +3057,11 @@ void launch_gather_ctl(hipStream_t st, const SysDev* d_sys, int nsys, int32_t* o
 {
     const int n = nsys * CTL_COUNT;
     hipLaunchKernelGGL(k_gather_ctl, dim3((n + 255) / 256), dim3(256), 0, st, d_sys, nsys, out);
+}
+
+void launch_gather_thermo(hipStream_t st, const SysDev* d_sys, int nsys, int nrec, ThermoDev* out)
+{
+    hipLaunchKernelGGL(k_gather_thermo, dim3((nsys * nrec + 255) / 256), dim3(256), 0, st, d_sys, nsys, nrec, out);
 }
 
 void launch_npt(hipStream_t st, const SysDev* d_sys, int nsys, const WorkItem* atom_work, int n_atom_work,

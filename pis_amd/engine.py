@@ -160,6 +160,12 @@ class Engine:
         check(lib().pis_sys_get_state(self._ptr, k, _dptr(pos), _dptr(vel), _dptr(force)))
         return pos, vel, force
 
+    def get_forces(self, k: int = 0) -> np.ndarray:
+        """Forces of system k alone (original order)."""
+        force = np.empty((self.specs[k].n, 3))
+        check(lib().pis_sys_get_state(self._ptr, k, None, None, _dptr(force)))
+        return force
+
     def get_positions(self, k: int = 0) -> np.ndarray:
         """Positions of system k alone (original order), for trajectory frames."""
         pos = np.empty((self.specs[k].n, 3))
@@ -351,8 +357,7 @@ class LJGpuManager:
         eng = self._engine_for(atoms)
         eng.set_state(0, atoms.positions, atoms.velocities, None)
         pe = float(eng.compute_potential()[0])
-        _, _, f = eng.get_state(0)
-        atoms.forces += f
+        atoms.forces += eng.get_forces(0)
         return pe
 
     def verlet_step_nve(self, atoms: Atoms, dt: float) -> float:
