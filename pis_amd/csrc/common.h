@@ -148,8 +148,8 @@ struct SysDev {
     double cellw[3];
     double half_skin2;     // (skin/2)^2
     double wslack;         // x-window slack of the list build: FP32 staging error + margin
-    // host-visible progress of a host-driven run (steps completed << 1 | a rebuild is due), null
-    // otherwise
+    // host-visible progress of a host-driven run (steps completed << 2 | kListDue or kStopped),
+    // null otherwise
     unsigned long long* progress;
     double dt, dt2;
     double kb, volume;
@@ -178,6 +178,8 @@ struct StepGate {
     int32_t step;
     int32_t fresh;
 };
+// the next step waits for a new list / the system froze (the barostat's box is too thin)
+constexpr unsigned kListDue = 1u, kStopped = 2u;
 
 // Cell numbering.  Cells are numbered tile-major: tiles in x-fastest order, and inside a
 // tile its cells in x-fastest order, so the atoms of a tile are contiguous after the sort.

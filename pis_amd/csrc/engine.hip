@@ -1018,6 +1018,7 @@ static pis_status replan_tiles_for_halo(pis_ctx* c, uint32_t k, int staged)
     }
     nh.dev.dt = h.dev.dt;
     nh.dev.dt2 = h.dev.dt2;
+    nh.dev.progress = h.dev.progress;
     nh.thermo = h.thermo;
     nh.thermo_cap = h.thermo_cap;
     nh.dev.thermo = h.thermo;
@@ -1241,7 +1242,7 @@ static pis_status batch_compute(pis_ctx* c, pis_thermo* out /* [nsys] or null */
 static pis_status enqueue_one(pis_ctx* c, bool first, bool record, bool nvt, bool timed, bool npt = false)
 {
     const int ns = (int)c->sys.size();
-    if (nvt && (first || npt)) launch_nhc_pre(c->stream, c->d_sys, ns);
+    if (nvt && (first || npt)) launch_nhc_pre(c->stream, c->d_sys, ns, StepGate{-1, 0});
     if (first || nvt) launch_integrate_pos(c->stream, c->d_sys, c->d_atom_work, c->n_atom_work, StepGate{-1, 0});
     launch_rebuild_sort(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work);
     if (timed) {
@@ -1297,36 +1298,44 @@ pis_status pis::enqueue_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
     return PIS_OK;
 }
 
-// nsteps of NVE (or NVT) of a context's only system, driven by the host: a step is its force
-// and reduction (and NVT's position update), and the five list-rebuild kernels are launched
+// nsteps of NVE, NVT or NPT of a context's only system, driven by the host: a step is its force
+// and reduction (and NVT's position update, and the barostat's launches around it), and the five list-rebuild kernels are launched
 // only when a step reports that the skin check fired, instead of in every step of a fixed
 // sequence (they cost 17 us of a 240 us step at 1M atoms even when they return at once, and
 // half of the step at 4000).  The step's progress arrives in a word of pinned memory; up to
 // `ahead` steps are queued beyond the last one known to be done, and those queued behind a
 // due rebuild find themselves gated off (StepGate) and are queued again behind it.
-static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt)
+static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt, bool npt)
 {
     constexpr uint64_t ahead = 3;
     volatile unsigned long long* word = c->progress;
     *word = 0;
     auto step = [&](uint64_t k, bool position, bool fresh) -> pis_status {
         const StepGate gate{(int32_t)k, fresh ? 1 : 0};
+        const int rec = record ? 1 : 0;
+        if (position && npt) {
+            launch_npt(c->stream, c->d_sys, 1, c->d_atom_work, c->n_atom_work, 1, rec, gate);
+            launch_nhc_pre(c->stream, c->d_sys, 1, gate);
+        }
         if (position) launch_integrate_pos(c->stream, c->d_sys, c->d_atom_work, c->n_atom_work, gate);
         if (fresh) launch_rebuild_sort(c->stream, c->d_sys, 1, c->d_atom_work, c->n_atom_work);
         PIS_TRY(enqueue_classes(c, fresh, 1, gate));
-        launch_reduce(c->stream, c->d_sys, 1, 1, record ? 1 : 0, 1, gate);
+        launch_reduce(c->stream, c->d_sys, 1, 1, rec, 1, gate);
+        if (npt)  // once the step itself is done
+            launch_npt(c->stream, c->d_sys, 1, c->d_atom_work, c->n_atom_work, 2, rec, StepGate{(int32_t)k + 1, 0});
         return PIS_OK;
     };
-    if (nvt) launch_nhc_pre(c->stream, c->d_sys, 1);
+    if (nvt && !npt) launch_nhc_pre(c->stream, c->d_sys, 1, StepGate{-1, 0});
     PIS_TRY(step(0, true, false));
     uint64_t queued = 1, done = 0;
     int64_t listed = -1;  // the last step queued with a rebuild
     for (unsigned idle = 0; done < nsteps;) {
         while (queued < nsteps && queued < done + ahead) PIS_TRY(step(queued++, nvt, false));
         const unsigned long long now = *word;
-        if ((now >> 1) > done) idle = 0;
-        done = now >> 1;
-        if ((now & 1) && done < nsteps && listed < (int64_t)done) {
+        if (now & kStopped) return PIS_OK;  // the caller finds the control words saying why
+        if ((now >> 2) > done) idle = 0;
+        done = now >> 2;
+        if ((now & kListDue) && done < nsteps && listed < (int64_t)done) {
             // step `done` waits for a new list, and what is queued behind it does nothing
             PIS_TRY(step(done, false, true));
             listed = (int64_t)done;
@@ -1338,7 +1347,7 @@ static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
             PIS_HIP(hipGetLastError());
             const hipError_t e = hipStreamQuery(c->stream);
             (void)hipGetLastError();  // "not ready" is no error of this run
-            if (e != hipErrorNotReady && *word == now && !((now & 1) && listed < (int64_t)done)) {
+            if (e != hipErrorNotReady && *word == now && !((now & kListDue) && listed < (int64_t)done)) {
                 if (e != hipSuccess) return fail(PIS_ERR_HIP, std::string("run: ") + hipGetErrorString(e));
                 return fail(PIS_ERR_HIP, "the run stopped after " + std::to_string(done) + " steps");
             }
@@ -1389,6 +1398,7 @@ static pis_status replan_for_box(pis_ctx* c, uint32_t k)
     // (whose list reference is void until the list is rebuilt in the new grid)
     nh.dev.dt = h.dev.dt;
     nh.dev.dt2 = h.dev.dt2;
+    nh.dev.progress = h.dev.progress;
     nh.dev.nhc_on = h.dev.nhc_on;
     nh.dev.npt_on = h.dev.npt_on;
     nh.thermo = h.thermo;
@@ -1430,7 +1440,7 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
     // NPT runs in chunks of kNptChunk steps: a system whose box would become thinner than
     // its cell grid freezes on the device, and the host re-plans it between chunks.
     c->listed = false;
-    const bool driven = c->sys.size() == 1 && !npt && !c->timing;
+    const bool driven = c->sys.size() == 1 && !c->timing;
     if (driven && !c->progress) {
         void* p = nullptr;
         PIS_HIP(hipHostMalloc(&p, 64, hipHostMallocDefault));
@@ -1462,14 +1472,18 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
             const int rec = out != nullptr ? 1 : 0;
             for (uint64_t t = 0; t < k; ++t) {
                 if (done + t == 0 || (resumed && t == 0))
-                    launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 0, rec);
-                launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 1, rec);
+                    launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 0, rec, StepGate{-1, 0});
+                if (driven) {
+                    PIS_TRY(drive_steps(c, k, out != nullptr, true, true));
+                    break;
+                }
+                launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 1, rec, StepGate{-1, 0});
                 PIS_TRY(enqueue_one(c, t == 0, out != nullptr, true, false, true));
-                launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 2, rec);
+                launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 2, rec, StepGate{-1, 0});
                 if ((t & 63) == 0) PIS_HIP(hipGetLastError());
             }
         } else if (driven) {
-            PIS_TRY(drive_steps(c, k, out != nullptr, nvt));
+            PIS_TRY(drive_steps(c, k, out != nullptr, nvt, false));
         } else {
             PIS_TRY(enqueue_steps(c, k, out != nullptr, nvt));
         }

@@ -31,7 +31,7 @@ void launch_gather_ctl(hipStream_t st, const SysDev* d_sys, int nsys, int32_t* o
 // Thermo records of every system, [nrec][nsys].
 void launch_gather_thermo(hipStream_t st, const SysDev* d_sys, int nsys, int nrec, ThermoDev* out);
 // NVT: start-of-step chain update and velocity scale; reset of the run's step counter.
-void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys);
+void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys, StepGate gate);
 void launch_nhc_run(hipStream_t st, const SysDev* d_sys, int nsys, uint64_t step0, uint64_t total);
 void launch_flip(hipStream_t st, const SysDev* d_sys, int nsys);
 // copy the live set's types and original indices into the other set (after a host sort)
@@ -39,7 +39,7 @@ void launch_sync_labels(hipStream_t st, const SysDev* d_sys, const WorkItem* ato
 // NPT around one NVT step: what = 0 start-of-step tensor sums, 1 barostat + box update and
 // scaled state, 2 end-of-step scaling, momentum update and thermo record (record != 0).
 void launch_npt(hipStream_t st, const SysDev* d_sys, int nsys, const WorkItem* atom_work, int n_atom_work,
-                int what, int record);
+                int what, int record, StepGate gate);
 void launch_list_to_orig(hipStream_t st, const SysDev* d_sys, const WorkItem* tile_work,
                          int n_tile_work, int scap, uint32_t* out, uint32_t* counts);
 

@@ -557,10 +557,10 @@ __device__ __forceinline__ bool step_runs(const StepGate& gate, int done, int re
 }
 
 // The run's progress for the host that drives it: one 8-byte store, nothing else is read by it.
-__device__ __forceinline__ void tell_progress(const SysDev& s, int done, bool due)
+__device__ __forceinline__ void tell_progress(const SysDev& s, int done, unsigned how)
 {
     if (s.progress)
-        __hip_atomic_store(s.progress, ((unsigned long long)done << 1) | (due ? 1ull : 0ull), __ATOMIC_RELAXED,
+        __hip_atomic_store(s.progress, ((unsigned long long)done << 2) | how, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -1995,7 +1995,7 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
     if (integrate && c_left == 0) return;  // frozen system: the whole block leaves
     if (!step_runs(gate, c_done, c_rb)) {
         // the host learns of a list that is due (NVT's position update found it) here
-        if (blockIdx.x == 0 && threadIdx.x == 0 && c_done == gate.step) tell_progress(s, c_done, true);
+        if (blockIdx.x == 0 && threadIdx.x == 0 && c_done == gate.step) tell_progress(s, c_done, kListDue);
         return;
     }
     // read set: the live set, or the freshly sorted one on a rebuild step; a step writes
@@ -2277,19 +2277,18 @@ __device__ __forceinline__ void sum_partials(const SysDev& s, double* v, double*
     block_sum4(v, rtmp);
 }
 
-__device__ void sum_tens(const SysDev& s, double* v, double* tmp);
 __device__ double sum_tens_ke(const SysDev& s, double* tmp);
 
 // Start of an NVT step (potential.rs:41-45): KE of the current velocities (the last
 // force launch's partials), chain forces and half step, and the velocity scale.  Launched
 // on a call's first NVT step and on every NPT step; k_reduce does it for the other NVT
 // steps at the end of the step before.
-__global__ __launch_bounds__(1024) void k_nhc_pre(const SysDev* __restrict__ sys)
+__global__ __launch_bounds__(1024) void k_nhc_pre(const SysDev* __restrict__ sys, StepGate gate)
 {
     __shared__ double rtmp[64];
     const SysDev& s = sys[blockIdx.x];
     __shared__ double ttmp[1024 + TENS_COUNT];
-    if (!s.nhc_on || s.ctl[CTL_LEFT] == 0) return;
+    if (!s.nhc_on || s.ctl[CTL_LEFT] == 0 || (gate.step >= 0 && s.ctl[CTL_DONE] != gate.step)) return;
     double ke;
     if (s.npt_on) {
         // NPT: the barostat rescaled the velocities since the last force launch; their KE
@@ -2352,10 +2351,17 @@ __device__ void mat3_exp(const double* a, double* out)
     e[0] = e[4] = e[8] = t[0] = t[4] = t[8] = 1.0;
     for (int j = 1; j <= 18; ++j) {
         mat3_mul(t, x, t);
+        double tmax = 0.0, emin = INFINITY;
         for (int k = 0; k < 9; ++k) {
             t[k] = t[k] / (double)j;
             e[k] = e[k] + t[k];
+            tmax = fmax(tmax, fabs(t[k]));
+            emin = fmin(emin, fabs(e[k]));
         }
+        // |x|_1 <= 1/2, so every element of every later term is below tmax / 2: once that is under
+        // a quarter ulp of every element of e, the rest of the series cannot change a bit (a
+        // barostat's steps get here after 4 or 5 of the 18 terms)
+        if (tmax < 0x1p-55 * emin) break;
     }
     for (int q = 0; q < sq; ++q) mat3_mul(e, e, e);
     for (int k = 0; k < 9; ++k) out[k] = e[k];
@@ -2397,20 +2403,20 @@ __device__ void symmetrize3(const double* a, double* out)
 }
 
 // delta_momentum (npt.rs:44-49): symmetrize((P - P0) * (V * 0.5 * dt)), P = (K + W) / V
-__device__ void mtk_add_delta(const double* sums, double* npt, double vol, double dt)
+__device__ void mtk_add_delta(const double* sums, double* mom, const double* target, double vol, double dt)
 {
     double d[9];
     const double f = vol * 0.5 * dt;
-    for (int k = 0; k < 9; ++k) d[k] = ((sums[TENS_K + k] + sums[TENS_W + k]) / vol - npt[NPT_TARGET + k]) * f;
+    for (int k = 0; k < 9; ++k) d[k] = ((sums[TENS_K + k] + sums[TENS_W + k]) / vol - target[k]) * f;
     symmetrize3(d, d);
-    for (int k = 0; k < 9; ++k) npt[NPT_MOM + k] += d[k];
+    for (int k = 0; k < 9; ++k) mom[k] += d[k];
 }
 
 // MTKBarostat::scale (npt.rs:51-58): exp(symmetrize(momentum / w) * factor * dt)
-__device__ void mtk_scale(const double* npt, double dt, double factor, double* out)
+__device__ void mtk_scale(const double* mom, double w, double dt, double factor, double* out)
 {
     double eta[9], a[9];
-    for (int k = 0; k < 9; ++k) eta[k] = npt[NPT_MOM + k] / npt[NPT_W];
+    for (int k = 0; k < 9; ++k) eta[k] = mom[k] / w;
     symmetrize3(eta, eta);
     for (int k = 0; k < 9; ++k) a[k] = eta[k] * factor * dt;
     mat3_exp(a, out);
@@ -2438,7 +2444,8 @@ __device__ double sum_tens_ke(const SysDev& s, double* tmp /* [blockDim.x] */)
     return tmp[0];
 }
 
-__device__ void sum_tens(const SysDev& s, double* v, double* tmp /* [blockDim.x + TENS_COUNT] */)
+// Fixed-order sums of every component, in tmp[blockDim.x + k] for all threads.
+__device__ void sum_tens(const SysDev& s, double* tmp /* [blockDim.x + TENS_COUNT] */)
 {
     // the partials read as one flat array, coalesced: with a stride that is a multiple of
     // TENS_COUNT every thread keeps one component; a fixed order of additions
@@ -2463,8 +2470,6 @@ __device__ void sum_tens(const SysDev& s, double* v, double* tmp /* [blockDim.x 
         tmp[blockDim.x + t] = x;
     }
     __syncthreads();
-    if (t == 0)
-        for (int k = 0; k < TENS_COUNT; ++k) v[k] = tmp[blockDim.x + k];
 }
 
 // Per 256-atom block of an NPT system: phase NPT_SUMS sums v v^T (kinetic_tensor, no
@@ -2475,14 +2480,15 @@ __device__ void sum_tens(const SysDev& s, double* v, double* tmp /* [blockDim.x 
 enum { NPT_SUMS = 0, NPT_BEGIN = 1, NPT_END = 2 };
 
 __global__ __launch_bounds__(kAtomThreads) void k_npt_atoms(const SysDev* __restrict__ sys,
-                                                             const WorkItem* __restrict__ work, int phase)
+                                                             const WorkItem* __restrict__ work, int phase,
+                                                             StepGate gate)
 {
     static_assert(kAtomThreads == 256, "the block sums below split 256 values into 8 x 32");
     __shared__ double red[10 * (kAtomThreads + 1)];
     __shared__ double red2[8 * 10];
     const WorkItem w = work[blockIdx.x];
     const SysDev& s = sys[w.sys];
-    if (!s.npt_on || s.ctl[CTL_LEFT] == 0) return;
+    if (!s.npt_on || s.ctl[CTL_LEFT] == 0 || (gate.step >= 0 && s.ctl[CTL_DONE] != gate.step)) return;
     const int a = w.idx + threadIdx.x;
     const State st = s.st[__builtin_amdgcn_readfirstlane(s.ctl[CTL_CUR])];
     double v[TENS_COUNT];
@@ -2559,26 +2565,32 @@ __global__ __launch_bounds__(kAtomThreads) void k_npt_atoms(const SysDev* __rest
 // within the cutoff (the reference finds pairs afresh in every force call).  A new box
 // thinner than the planned cell grid raises CTL_BOX and freezes the system before anything
 // of the step is applied (the host re-plans the grid and resumes from that step).
-__global__ __launch_bounds__(1024) void k_npt_begin(const SysDev* __restrict__ sys)
+__global__ __launch_bounds__(1024) void k_npt_begin(const SysDev* __restrict__ sys, StepGate gate)
 {
     __shared__ double tmp[1024 + TENS_COUNT];
+    __shared__ double mom[9], scaled[2][9];
     const SysDev& s = sys[blockIdx.x];
-    if (!s.npt_on || s.ctl[CTL_LEFT] == 0) return;
-    double v[TENS_COUNT];
-    sum_tens(s, v, tmp);
-    if (threadIdx.x != 0) return;
+    if (!s.npt_on || s.ctl[CTL_LEFT] == 0 || (gate.step >= 0 && s.ctl[CTL_DONE] != gate.step)) return;
     double* npt = s.npt;
     double* box = s.box;
-    // the step's barostat update on a copy, committed only when the new box still fits
-    // the planned cell grid
-    double nl[NPT_COUNT];
-    for (int k = 0; k < NPT_COUNT; ++k) nl[k] = npt[k];
-    mtk_add_delta(v, nl, box[BOX_VOL], s.dt);
-    mtk_scale(nl, s.dt, -0.5, nl + NPT_SCALE);
-    double sh[9], h[9], hi[9];
-    mtk_scale(nl, s.dt, 1.0, sh);
-    for (int k = 0; k < 9; ++k) nl[NPT_HINV_OLD + k] = box[BOX_HINV + k];
-    mat3_mul(sh, box + BOX_H, h);
+    sum_tens(s, tmp);
+    // The two matrix exponentials, each a chain of hundreds of dependent operations, on one lane
+    // of a wave of its own.  The step's barostat update stays on a copy, committed only when
+    // the new box still fits the planned cell grid.
+    if (threadIdx.x == 0 || threadIdx.x == 64) {
+        double m[9], out[9];
+        for (int k = 0; k < 9; ++k) m[k] = npt[NPT_MOM + k];
+        mtk_add_delta(tmp + 1024, m, npt + NPT_TARGET, box[BOX_VOL], s.dt);
+        mtk_scale(m, npt[NPT_W], s.dt, threadIdx.x == 0 ? -0.5 : 1.0, out);
+        for (int k = 0; k < 9; ++k) {
+            scaled[threadIdx.x / 64][k] = out[k];
+            if (threadIdx.x == 0) mom[k] = m[k];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    double h[9], hi[9];
+    mat3_mul(scaled[1], box + BOX_H, h);
     mat3_inverse(h, hi);
     const double vol = fabs(mat3_det(h));
     if (s.mode != MODE_WHOLE) {
@@ -2586,17 +2598,20 @@ __global__ __launch_bounds__(1024) void k_npt_begin(const SysDev* __restrict__ s
             const double* p = h + 3 * ((k + 1) % 3);
             const double* q = h + 3 * ((k + 2) % 3);
             const double cx = p[1] * q[2] - p[2] * q[1], cy = p[2] * q[0] - p[0] * q[2], cz = p[0] * q[1] - p[1] * q[0];
-            if (!(vol / sqrt(cx * cx + cy * cy + cz * cz) >= nl[NPT_RCL] * (double)s.nc[k])) {
+            if (!(vol / sqrt(cx * cx + cy * cy + cz * cz) >= npt[NPT_RCL] * (double)s.nc[k])) {
                 // too thin for the cell grid: nothing of this step is applied and the system
                 // freezes (every later kernel skips it) until the host re-plans the grid
                 s.ctl[CTL_BOX] = 1;
                 s.ctl[CTL_LEFT] = 0;
+                tell_progress(s, s.ctl[CTL_DONE], kStopped);
                 return;
             }
         }
     }
-    for (int k = 0; k < NPT_COUNT; ++k) npt[k] = nl[k];
     for (int k = 0; k < 9; ++k) {
+        npt[NPT_MOM + k] = mom[k];
+        npt[NPT_SCALE + k] = scaled[0][k];
+        npt[NPT_HINV_OLD + k] = box[BOX_HINV + k];
         box[BOX_H + k] = h[k];
         box[BOX_HINV + k] = hi[k];
     }
@@ -2627,18 +2642,18 @@ __global__ __launch_bounds__(1024) void k_npt_begin(const SysDev* __restrict__ s
 // second momentum update; the step's thermo record gets the KE, temperature and pressure
 // of the final velocities and the NPT Hamiltonian (simulation.rs:106-114): PE + KE + chain
 // KE + chain PE (0: eta never moves) + barostat KE (npt.rs:60-62) + barostat PE (npt.rs:64-66).
-__global__ __launch_bounds__(1024) void k_npt_end(const SysDev* __restrict__ sys, int record)
+__global__ __launch_bounds__(1024) void k_npt_end(const SysDev* __restrict__ sys, int record, StepGate gate)
 {
     __shared__ double tmp[1024 + TENS_COUNT];
     const SysDev& s = sys[blockIdx.x];
-    if (!s.npt_on || s.ctl[CTL_LEFT] == 0) return;
-    double v[TENS_COUNT];
-    sum_tens(s, v, tmp);
+    if (!s.npt_on || s.ctl[CTL_LEFT] == 0 || (gate.step >= 0 && s.ctl[CTL_DONE] != gate.step)) return;
+    sum_tens(s, tmp);
     if (threadIdx.x != 0) return;
+    const double* v = tmp + 1024;
     double* npt = s.npt;
     const double* box = s.box;
     const double vol = box[BOX_VOL];
-    mtk_add_delta(v, npt, vol, s.dt);
+    mtk_add_delta(v, npt + NPT_MOM, npt + NPT_TARGET, vol, s.dt);
     const int k = s.ctl[CTL_STEP] - 1;
     if (!record || k < 0 || k >= s.thermo_cap) return;
     const double* m = npt + NPT_MOM;
@@ -2736,7 +2751,7 @@ __global__ __launch_bounds__(1024) void k_reduce(const SysDev* __restrict__ sys,
         if (c_remain > 0) ctl[CTL_REMAIN] = c_remain - 1;
         if (c_left > 0) ctl[CTL_LEFT] = c_left - 1;
         ctl[CTL_DONE] = c_done + 1;
-        tell_progress(s, c_done + 1, c_next != 0);
+        tell_progress(s, c_done + 1, c_next ? kListDue : 0u);
     } else if (flip && c_rb) {
         ctl[CTL_CUR] = c_cur ^ 1;
         ctl[CTL_REBUILD] = 0;
@@ -3042,9 +3057,9 @@ void launch_reduce(hipStream_t st, const SysDev* d_sys, int nsys, int flip, int 
     hipLaunchKernelGGL(k_reduce, dim3(nsys), dim3(1024), 0, st, d_sys, flip, record, step, gate);
 }
 
-void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys)
+void launch_nhc_pre(hipStream_t st, const SysDev* d_sys, int nsys, StepGate gate)
 {
-    hipLaunchKernelGGL(k_nhc_pre, dim3(nsys), dim3(1024), 0, st, d_sys);
+    hipLaunchKernelGGL(k_nhc_pre, dim3(nsys), dim3(1024), 0, st, d_sys, gate);
 }
 
 void launch_nhc_run(hipStream_t st, const SysDev* d_sys, int nsys, uint64_t step0, uint64_t total)
@@ -3065,17 +3080,17 @@ void launch_gather_thermo(hipStream_t st, const SysDev* d_sys, int nsys, int nre
 }
 
 void launch_npt(hipStream_t st, const SysDev* d_sys, int nsys, const WorkItem* atom_work, int n_atom_work,
-                int what, int record)
+                int what, int record, StepGate gate)
 {
     // what: 0 start-of-step sums, 1 start (barostat, box, scaled state), 2 end of the step
     if (what == 0) {
-        hipLaunchKernelGGL(k_npt_atoms, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, (int)NPT_SUMS);
+        hipLaunchKernelGGL(k_npt_atoms, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, (int)NPT_SUMS, gate);
     } else if (what == 1) {
-        hipLaunchKernelGGL(k_npt_begin, dim3(nsys), dim3(1024), 0, st, d_sys);
-        hipLaunchKernelGGL(k_npt_atoms, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, (int)NPT_BEGIN);
+        hipLaunchKernelGGL(k_npt_begin, dim3(nsys), dim3(1024), 0, st, d_sys, gate);
+        hipLaunchKernelGGL(k_npt_atoms, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, (int)NPT_BEGIN, gate);
     } else {
-        hipLaunchKernelGGL(k_npt_atoms, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, (int)NPT_END);
-        hipLaunchKernelGGL(k_npt_end, dim3(nsys), dim3(1024), 0, st, d_sys, record);
+        hipLaunchKernelGGL(k_npt_atoms, dim3(n_atom_work), dim3(kAtomThreads), 0, st, d_sys, atom_work, (int)NPT_END, gate);
+        hipLaunchKernelGGL(k_npt_end, dim3(nsys), dim3(1024), 0, st, d_sys, record, gate);
     }
 }
 

@@ -4,7 +4,8 @@ the same bits, records and rebuild counts.
 
 The cases are the edges of the drive: runs shorter than the steps queued ahead, a skin so
 thin that nearly every step rebuilds, no skin at all, a rebuild due in a call's first step,
-runs continued over several calls, and NVT (whose position update finds the due rebuild)."""
+runs continued over several calls, NVT (whose position update finds the due rebuild) and NPT
+(whose second half runs behind the step)."""
 import numpy as np
 import pytest
 
@@ -20,30 +21,33 @@ def spec_with(skin, n=1372, temp=1.5):
     return s
 
 
-def run(specs, precision, calls, nvt):
+def run(specs, precision, calls, ens):
     with Engine(specs, precision) as eng:
         eng.load()
         eng.compute_potential()
-        if nvt:
+        if ens == "nvt":
             eng.nvt_init(1.5, 1.0, 2.0)
+        if ens == "npt":
+            eng.npt_init(1.5, 1.0, 2.0, 1.0, 30.0)
         th = []
         done = 0
         for k in calls:
-            th.append(eng.run_nvt(0.005, k, ramp=(done, sum(calls))) if nvt else eng.run_nve(0.005, k))
+            step = {"nve": eng.run_nve, "nvt": eng.run_nvt, "npt": eng.run_npt}[ens]
+            th.append(step(0.005, k) if ens == "nve" else step(0.005, k, ramp=(done, sum(calls))))
             done += k
         return np.concatenate(th)[:, 0], eng.get_state(0), eng.stats()["rebuilds"] // len(specs)
 
 
-@pytest.mark.parametrize("nvt", [False, True], ids=["nve", "nvt"])
+@pytest.mark.parametrize("ens", ["nve", "nvt", "npt"])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("skin,calls", [(0.3, [1]), (0.3, [2, 1]), (0.3, [3, 4, 5]), (0.3, [60]), (0.02, [1, 2, 20]),
                                         (0.0, [7]), (0.15, [31, 1, 1, 17])],
                          ids=lambda v: str(v))
-def test_driven_run_equals_the_fixed_sequence(skin, calls, precision, nvt):
+def test_driven_run_equals_the_fixed_sequence(skin, calls, precision, ens):
     spec = spec_with(skin)
-    th1, st1, r1 = run([spec], precision, calls, nvt)
-    th2, st2, r2 = run([spec, spec], precision, calls, nvt)
-    print(f"skin {skin} calls {calls} {precision} nvt={nvt}: {r1} rebuilds", flush=True)
+    th1, st1, r1 = run([spec], precision, calls, ens)
+    th2, st2, r2 = run([spec, spec], precision, calls, ens)
+    print(f"skin {skin} calls {calls} {precision} {ens}: {r1} rebuilds", flush=True)
     assert np.array_equal(th1, th2)
     for a, b in zip(st1, st2):
         assert np.array_equal(a, b)
