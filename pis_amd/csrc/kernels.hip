@@ -1513,6 +1513,10 @@ struct Acc32 {
 // take four.  It is zeroed for a candidate outside the cutoff (raw staging masks padding
 // entries by count, tile-relative staging puts the padding slot kPadFar away, so its r^2 is
 // finite in FP64 and fails the cutoff), and every power and product of it is then zero.
+// Bound by FP64 issue and latency: with one mask instead of one per term and the sums below,
+// the FP64 force kernel needs 167 registers (206 before), so 3 waves per SIMD instead of 2;
+// 1,048,576 atoms took 228 us, 192 us with this and 172 us with the parameters of a lone
+// species read once per workgroup as well.
 __device__ __forceinline__ double masked_inverse(double r2, bool in)
 {
     const double x = __builtin_amdgcn_rcp(r2);
@@ -1971,7 +1975,8 @@ __device__ __forceinline__ double pick3(int c, double x, double y, double z) { r
 // workgroups per tile, each with 64 of every 256 of the tile's atoms and four lanes per atom.
 // A lone small system leaves most of the chip idle, and its time is one workgroup's chain of
 // latencies: this cuts the chain of list groups and spreads the pairs over four times the
-// CUs, for four times the staging.  Both give the same bits.
+// CUs, for four times the staging.  Both give the same bits.  FP64 force launch, KL = 1 / 4:
+// 500 atoms 28.7 / 10.5 us, 4000 atoms 31 / 17 us; list build 103 / 24 and 108 / 45 us.
 template <int SCAP, bool MIXED, int KIND, int KL>
 __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value)) void k_force(
     const SysDev* __restrict__ sys, const WorkItem* __restrict__ tiles, int ntw, int integrate, StepGate gate)
@@ -2565,6 +2570,8 @@ __global__ __launch_bounds__(kAtomThreads) void k_npt_atoms(const SysDev* __rest
 // within the cutoff (the reference finds pairs afresh in every force call).  A new box
 // thinner than the planned cell grid raises CTL_BOX and freezes the system before anything
 // of the step is applied (the host re-plans the grid and resumes from that step).
+// Bound by one lane's chain of 3x3 products: the two exponentials run on lanes of different
+// waves and stop once their series cannot change a bit (24 -> 10 us at 32,000 atoms).
 __global__ __launch_bounds__(1024) void k_npt_begin(const SysDev* __restrict__ sys, StepGate gate)
 {
     __shared__ double tmp[1024 + TENS_COUNT];
