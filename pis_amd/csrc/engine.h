@@ -157,8 +157,8 @@ struct pis_ctx {
 
 namespace pis {
 
-// Device memory of one system (one allocation, carved) and its tables.
-pis_status alloc_system(SysHost& h);
+// Device memory of one system (one allocation, carved) and its tables, filled on `st`.
+pis_status alloc_system(SysHost& h, hipStream_t st);
 // Every system's descriptor to the device copy the kernels read.
 pis_status upload_sys(pis_ctx* c);
 void free_ctx(pis_ctx* c);
