@@ -146,6 +146,7 @@ struct pis_ctx {
     bool snap_pending = false;
     // host-driven runs of a single system: the progress word its steps write (pinned)
     unsigned long long* progress = nullptr;
+    bool late = false;  // the last run's thread was kept off its CPU near the run's end
     // statistics / timing
     uint64_t steps = 0, force_launches = 0;
     bool timing = false;

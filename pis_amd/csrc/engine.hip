@@ -1295,15 +1295,27 @@ pis_status pis::enqueue_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
 }
 
 // nsteps of NVE, NVT or NPT of a context's only system, driven by the host: a step is its force
-// and reduction (and NVT's position update, and the barostat's launches around it), and the five list-rebuild kernels are launched
-// only when a step reports that the skin check fired, instead of in every step of a fixed
-// sequence (they cost 17 us of a 240 us step at 1M atoms even when they return at once, and
-// half of the step at 4000).  The step's progress arrives in a word of pinned memory; up to
-// `ahead` steps are queued beyond the last one known to be done, and those queued behind a
-// due rebuild find themselves gated off (StepGate) and are queued again behind it.
+// and reduction (and NVT's position update, and the barostat's launches around it), and the
+// five list-rebuild kernels are launched only when a step reports that the skin check fired,
+// instead of in every step of a fixed sequence (they cost 17 us of a 240 us step at 1M atoms
+// even when they return at once, and half of the step at 4000).  The step's progress arrives
+// in a word of pinned memory; up to `ahead` steps are queued beyond the last one known to be
+// done, and those queued behind a due rebuild find themselves gated off (StepGate) and are
+// queued again behind it.
+//
+// All of that needs this thread on a CPU whenever a rebuild comes due (every 8 steps at 1M
+// atoms).  A thread that lost its CPU for longer than kLate (the scheduler's slices are
+// milliseconds) is on a busy host, and queues the next `burst` steps whole, with their rebuild
+// launches: they need no answer.  The switch waits for a known state, all lean steps done or
+// one found due, since a lean step may have done part of its work.  Beside 16 / 32 busy
+// processes on 16 CPUs a step takes 220 / 220 us at 1,048,576 atoms (without this 368 / 540, the
+// fixed sequence 230 / 240, alone 200) and 51 / 66 us at 131,072 (84 / 86, 55 / 60, 42); with
+// bursts of 256 steps, which a slice outlasts at small sizes, 60 / 80.
 static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt, bool npt)
 {
-    constexpr uint64_t ahead = 3;
+    using Clock = std::chrono::steady_clock;
+    constexpr uint64_t ahead = 3, burst = 1024;
+    constexpr std::chrono::microseconds kLate(500);
     volatile unsigned long long* word = c->progress;
     *word = 0;
     auto step = [&](uint64_t k, bool position, bool fresh) -> pis_status {
@@ -1322,11 +1334,31 @@ static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
         return PIS_OK;
     };
     if (nvt && !npt) launch_nhc_pre(c->stream, c->d_sys, 1, StepGate{-1, 0});
-    PIS_TRY(step(0, true, false));
+    bool late = c->late;  // a call that follows on a busy host starts with whole steps
+    PIS_TRY(step(0, true, late));
     uint64_t queued = 1, done = 0;
-    int64_t listed = -1;  // the last step queued with a rebuild
+    uint64_t whole = 0;              // steps below are queued with their rebuild launches
+    int64_t listed = late ? 0 : -1;  // the last step queued so
+    uint64_t calm = 0;               // end of the last stretch that a late thread asked for
+    c->late = false;
+    Clock::time_point seen = Clock::now();
     for (unsigned idle = 0; done < nsteps;) {
-        while (queued < nsteps && queued < done + ahead) PIS_TRY(step(queued++, nvt, false));
+        if (late && (queued == done || (int64_t)queued == listed + 1)) {
+            whole = done + burst;
+            late = false;
+        }
+        const uint64_t before = queued;
+        for (; queued < nsteps && (queued < whole || (!late && queued < done + ahead)); ++queued) {
+            const bool fresh = queued < whole;
+            PIS_TRY(step(queued, nvt, fresh));
+            if (fresh) listed = (int64_t)queued;
+        }
+        const Clock::time_point t = Clock::now();
+        if (queued == before && t - seen > kLate) {
+            late = true;
+            calm = done + burst;
+        }
+        seen = t;
         const unsigned long long now = *word;
         if (now & kStopped) return PIS_OK;  // the caller finds the control words saying why
         if ((now >> 2) > done) idle = 0;
@@ -1337,19 +1369,21 @@ static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
             listed = (int64_t)done;
             queued = done + 1;
             idle = 0;
+            seen = Clock::now();
         } else if (++idle == 1u << 16) {
             // nothing for milliseconds: a stream that has run dry will not move any more
             idle = 0;
             PIS_HIP(hipGetLastError());
             const hipError_t e = hipStreamQuery(c->stream);
             (void)hipGetLastError();  // "not ready" is no error of this run
-            if (e != hipErrorNotReady && *word == now && !((now & kListDue) && listed < (int64_t)done)) {
+            if (e != hipErrorNotReady && *word == now) {
                 if (e != hipSuccess) return fail(PIS_ERR_HIP, std::string("run: ") + hipGetErrorString(e));
                 return fail(PIS_ERR_HIP, "the run stopped after " + std::to_string(done) + " steps");
             }
         }
         __builtin_ia32_pause();
     }
+    c->late = nsteps < calm;
     c->force_launches += nsteps;
     return PIS_OK;
 }
