@@ -136,7 +136,9 @@ struct pis_ctx {
     void* h_pin = nullptr;  // pinned staging of small transfers (at most kPinnedMax bytes)
     size_t pin_bytes = 0;
     std::vector<SysDev> sent;  // descriptors as last uploaded to d_sys
-    bool listed = false;  // the only system's list is known to be current (no rebuild pending)
+    // the only system's list is that of the state just uploaded: true from a successful
+    // sys_set_state to the next run, re-plan or change of the tiles
+    bool listed = false;
     // trajectory snapshots: positions copied on `stream`, sent to the host on snap_stream
     // (default priority) while later steps run; one in flight at a time
     hipStream_t snap_stream = nullptr;

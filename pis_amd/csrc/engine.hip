@@ -677,6 +677,7 @@ pis_status pis::group_tiles(pis_ctx* c)
         c->nlanes = nl;
     }
     for (auto& stale : c->graph_stale) stale = true;
+    c->listed = false;
     PIS_TRY(reserve_lanes(c, c->nlanes));
     c->n_tile_work = (int)tw.size();
     if (c->tile_work_cap < tw.size()) {
@@ -1536,6 +1537,7 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
                 c->steps += completed;
                 done += completed;
                 PIS_TRY(replan_for_box(c, 0));
+                c->listed = false;  // steps follow
                 resumed = true;
                 continue;
             }
