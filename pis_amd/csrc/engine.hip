@@ -1361,7 +1361,10 @@ static pis_status drive_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt
         }
         seen = t;
         const unsigned long long now = *word;
-        if (now & kStopped) return PIS_OK;  // the caller finds the control words saying why
+        if (now & kStopped) {  // the caller finds the control words saying why
+            c->force_launches += now >> 2;
+            return PIS_OK;
+        }
         if ((now >> 2) > done) idle = 0;
         done = now >> 2;
         if ((now & kListDue) && done < nsteps && listed < (int64_t)done) {

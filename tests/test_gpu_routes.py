@@ -113,6 +113,7 @@ def test_a_run_that_is_planned_again_on_the_way_has_every_record():
     assert np.abs(th - th2).max() <= 1e-8 * np.abs(th).max()
     assert abs(pe - th[-1, 0]) <= 1e-12 * abs(pe)  # the list that the run left behind is whole
     assert stats["steps"] == 120
+    assert stats["force_launches"] == 120 + 2  # a force launch a step, and the two force calls
 
 
 def state_of(n, seed):
