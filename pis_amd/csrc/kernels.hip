@@ -396,7 +396,7 @@ constexpr double kPadFar = 1e30;  // squared: 1e60, finite in FP64, +inf in FP32
 // with raw positions (a per-pair minimum image would fold it back) it sits at the origin
 // and the force loop masks those entries by count.
 // Returns the number of staged atoms (uniform over the block); > SCAP means overflow
-// and nothing was staged.  smap (SCAP + 1 bytes, may be null) receives the halo cell of
+// and nothing was staged.  smap (SCAP + 1 bytes, null with WIDE) receives the halo cell of
 // every slot, each cell's thread filling its run, so a slot finds its atom with one LDS
 // read instead of a binary search over the halo's cell offsets.  Staged coordinates are
 // multiplied by `scale` (1, or 1/sigma for the single-species mixed loop).
@@ -428,7 +428,8 @@ __device__ int stage_tile(const SysDev& s, const State& st, const TileGeom& g, d
     int total_staged = 0;
     if constexpr (WIDE) {
         // a half-wave per halo cell, every cell of a round in flight: no slot-to-cell map to
-        // fill and to search, at the price of idle lanes (a cell holds 19 to 32 atoms)
+        // fill and to search, at the price of idle lanes; the loop over i takes a cell of any
+        // population, in passes of 32
         if (ne > 1) {
             constexpr int R = 5;
             const int nh = (int)blockDim.x >> 5, h = tid >> 5, l = tid & 31;
@@ -451,7 +452,7 @@ __device__ int stage_tile(const SysDev& s, const State& st, const TileGeom& g, d
                     if (e >= ne) break;
                     const int p0 = pref[e], n = pref[e + 1] - p0;
                     for (int i = l; i < n; i += 32) {
-                        if (i != l) {  // a cell of more than 32 atoms
+                        if (i != l) {  // a pass after the first
                             const int a = ecell[e] + i;
                             x[r] = gbl(st.x)[a];
                             y[r] = gbl(st.y)[a];
@@ -1403,7 +1404,7 @@ __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_lis
     // slots past the padding slot take the candidate reads that run past a window's end.
     __shared__ float Px[SCAP + 1 + 64], Py[SCAP + 1 + 64], Pz[SCAP + 1 + 64];
     __shared__ uint8_t Pt[SCAP + 1 + 64];
-    __shared__ uint8_t smap[SCAP + 1];
+    __shared__ uint8_t smap[KL == 1 ? SCAP + 1 : 1];  // wide staging needs none
     __shared__ int pref[kMaxHalo + 1];
     __shared__ int ecell[kMaxHalo];
     __shared__ int stmp[16];
@@ -1425,7 +1426,7 @@ __global__ __launch_bounds__(kTileThreads, PIS_BUILD_MIN_WAVES) void k_build_lis
         tile_center(s, g, cx, cy, cz);
         for (int q = threadIdx.x; q < nt * nt; q += blockDim.x) ppl[q] = s.pp[q];
         const int total = stage_tile<SCAP, REL ? STAGE_REL : STAGE_RAW, float, (KL > 1)>(
-            s, st, g, cx, cy, cz, Px, Py, Pz, Pt, pref, ecell, stmp, smap);
+            s, st, g, cx, cy, cz, Px, Py, Pz, Pt, pref, ecell, stmp, KL == 1 ? smap : (uint8_t*)nullptr);
         if (threadIdx.x == 0) atomicMax(&s.ctl[CTL_MAXSTAGE], total);
         if (total > SCAP) {
             if (threadIdx.x == 0) atomicOr(&s.ctl[CTL_OVF_STAGE], 1);
