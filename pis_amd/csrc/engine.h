@@ -219,7 +219,7 @@ size_t system_bytes(const Plan& p, int thermo_records);
 // Enqueues `nsteps` steps (record: thermo per step; nvt: the chain is applied) of every
 // system on the context's stream, from captured graphs when use_graph is set; the first
 // step runs the position-update kernel, later NVE steps find their positions advanced by
-// the previous step's force kernel.
+// the previous step's force kernel.  The caller has set the systems' CTL_REMAIN to `nsteps`.
 pis_status enqueue_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt);
 
 }  // namespace pis

@@ -441,9 +441,12 @@ int pis::stage_class_for(double need) { return scap_for(need); }
 // one workgroup's chain of latencies; four lanes per atom and four workgroups per tile cut
 // that chain, for four times the halo staging.  Measured per step, one against four: 500
 // atoms (2 work items) 39 against 26 us, 4000 (18 tiles) 55 against 37, 40 Kob-Andersen
-// systems in classes of 2 to 500 tiles 354 against 288; 176 tiles break even in mixed
-// precision and lose in FP64 (95 against 110 us of an NPT step), 700 tiles lose (65 against
-// 122).  The line lies below the first loss.
+// systems in classes of 2 to 500 tiles 354 against 288.  Speedup by tiles, mixed / FP64: one
+// species 16-64 tiles 1.17-1.39 / 1.30-1.46, 81 1.09 / 1.18, 100 1.05 / 1.13, 144 0.95 / 0.86, 176
+// 0.97 / 0.83; two species 18-84 1.36-1.66 / 1.47-1.80, 125 1.27 / 1.45, 200 1.01 / 0.88; sheared boxes
+// 64 1.29 / 1.36, 100 1.16 / 1.23, 176 0.84 / 0.73; batches 32-120 1.32-1.77 / 1.43-1.82, 216 1.03 /
+// 0.98, 432 0.90 / 0.81.  The line lies between the last gain and the first loss, which are
+// near enough to each other in every kind for one line to serve all.
 #ifndef PIS_LANES_TILES
 #define PIS_LANES_TILES 128
 #endif
@@ -945,10 +948,10 @@ static pis_status check_ctl(pis_ctx* c, uint32_t k, const int32_t* ctl)
     return PIS_OK;
 }
 
-// After everything queued on the stream: the control words of every system [nsys][CTL_COUNT]
-// and, if `out`, nrec thermo records per system [nrec][nsys] into `out`, with one wait.  The
-// records stay in c->h_pin (out untouched) until the caller has looked at the flags; more than
-// fit there are left for read_thermo (*pinned false).
+// After everything queued on the stream, with one wait: the control words of every system
+// [nsys][CTL_COUNT] in `ctl`, and nrec thermo records per system [nrec][nsys] in c->h_pin behind
+// align256 of the words' bytes, for the caller to copy once it has looked at the flags.  Records
+// that do not fit there are left for read_thermo (*pinned false).
 static pis_status collect_run(pis_ctx* c, uint64_t nrec, std::vector<int32_t>& ctl, bool* pinned)
 {
     const size_t ns = c->sys.size(), nc = ns * CTL_COUNT * 4, nt = nrec * ns * sizeof(ThermoDev);
@@ -1221,7 +1224,6 @@ static pis_status batch_compute(pis_ctx* c, pis_thermo* out /* [nsys] or null */
     std::vector<int32_t> ctl;
     bool pinned;
     PIS_TRY(collect_run(c, 1, ctl, &pinned));
-    PIS_HIP(hipStreamSynchronize(c->stream));
     PIS_TRY(collect_timing(c));
     const size_t ns = c->sys.size();
     for (uint32_t k = 0; k < ns; ++k) PIS_TRY(check_ctl(c, k, &ctl[(size_t)k * CTL_COUNT]));
@@ -1231,11 +1233,11 @@ static pis_status batch_compute(pis_ctx* c, pis_thermo* out /* [nsys] or null */
     return PIS_OK;
 }
 
-// One step's launches; `first`: the position-update kernel runs (a call's first step,
-// and every NVT step, whose velocity scaling needs the chain update in between).
-// One step.  nvt: the Nose-Hoover chain wraps it; the chain's start-of-step update runs
-// as its own launch on a call's first step and on NPT steps (whose barostat rescaled the
-// velocities since), otherwise at the end of the previous step (k_reduce).
+// One step's launches.  `first`: a call's first step, which runs the position-update kernel, as
+// every NVT step does, whose velocity scaling needs the chain update in between.  nvt: the
+// Nose-Hoover chain wraps the step; the chain's start-of-step update runs as its own launch
+// on a call's first step and on NPT steps (whose barostat rescaled the velocities since),
+// otherwise at the end of the previous step (k_reduce).
 static pis_status enqueue_one(pis_ctx* c, bool first, bool record, bool nvt, bool timed, bool npt = false)
 {
     const int ns = (int)c->sys.size();
@@ -1256,8 +1258,6 @@ static pis_status enqueue_one(pis_ctx* c, bool first, bool record, bool nvt, boo
 
 pis_status pis::enqueue_steps(pis_ctx* c, uint64_t nsteps, bool record, bool nvt)
 {
-    const int ns = (int)c->sys.size();
-    launch_set_ctl(c->stream, c->d_sys, ns, CTL_REMAIN, (int)std::min<uint64_t>(nsteps, (uint64_t)INT32_MAX));
     if (c->use_graph && !c->timing) {
         for (int steady = 0; steady < 2; ++steady) {
             const int gi = (record ? 1 : 0) + (nvt ? 2 : 0) + 4 * steady;
@@ -1505,13 +1505,10 @@ static pis_status batch_run(pis_ctx* c, const double* dts, uint64_t nsteps, pis_
             // previous step ended with (nothing moves in between), so only a call's first
             // step, and the first after a re-plan, computes them.
             const int rec = out != nullptr ? 1 : 0;
-            for (uint64_t t = 0; t < k; ++t) {
-                if (done + t == 0 || (resumed && t == 0))
-                    launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 0, rec, StepGate{-1, 0});
-                if (driven) {
-                    PIS_TRY(drive_steps(c, k, out != nullptr, true, true));
-                    break;
-                }
+            if (done == 0 || resumed)
+                launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 0, rec, StepGate{-1, 0});
+            if (driven) PIS_TRY(drive_steps(c, k, out != nullptr, true, true));
+            for (uint64_t t = 0; t < k && !driven; ++t) {
                 launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 1, rec, StepGate{-1, 0});
                 PIS_TRY(enqueue_one(c, t == 0, out != nullptr, true, false, true));
                 launch_npt(c->stream, c->d_sys, ns, c->d_atom_work, c->n_atom_work, 2, rec, StepGate{-1, 0});

@@ -1970,7 +1970,7 @@ __device__ __forceinline__ double pick3(int c, double x, double y, double z) { r
 
 // KIND: one of KIND_ORTHO, KIND_TRI (tile-relative staging), KIND_ORTHO_RAW, KIND_TRI_RAW
 // (raw staging with a per-pair image).  Mixed precision with tile-relative staging stages
-// FP32 coordinates (atom_forces_f32); every other combination stages FP64.
+// FP32 coordinates (group_f32); every other combination stages FP64.
 //
 // KL = 1: a workgroup per tile, a lane per atom.  KL = 4 (small launches, see class_lanes): four
 // workgroups per tile, each with 64 of every 256 of the tile's atoms and four lanes per atom.

@@ -380,6 +380,7 @@ void worker_main(pis_server* sv)
         if (running) {
             pis_ctx* c = sv->ctx;
             launch_set_ctl(c->stream, c->d_sys, (int)c->sys.size(), CTL_STEP, 0);
+            launch_set_ctl(c->stream, c->d_sys, (int)c->sys.size(), CTL_REMAIN, (int)sv->round_steps);
             st = enqueue_steps(c, (uint64_t)sv->round_steps, true, false);
             if (st == PIS_OK) {
                 const hipError_t e = hipGetLastError();
