@@ -29,6 +29,8 @@ sys.path.insert(0, ROOT)
 
 METRIC = "atom-steps/s at 1M LJ atoms, FP64 vs FP32/FP64 mixed; p50/p99 job latency"
 HBM_PEAK_GBS = 8000.0
+# how a lone system's steps run, whatever the graph mode of its context
+STEPPING = "launched by the host step by step, list rebuilds when a step reports one due"
 
 
 def log(msg):
@@ -109,19 +111,19 @@ def drift_stats(etot, n):
     }
 
 
-def run_gpu(spec, precision, steps, warmup, graph, timing_steps=50):
+def run_gpu(spec, precision, steps, warmup, timing_steps=50):
     """The headline measurement: W warm-up steps with the timed call's own settings
-    (thermo recorded every step, graph mode as timed), so the thermo ring and the captured
-    step graphs exist before t0; then exactly K steps timed with kernel timing off.  The
-    force kernel's launch time comes from a separate pass with HIP events around each force
-    launch on the context's stream."""
+    (thermo recorded every step), so the thermo ring exists before t0; then exactly K steps
+    timed with kernel timing off.  A lone system's steps are launched by the host, the list's
+    rebuild only when a step reports it due.  The force kernel's launch time comes from a
+    separate pass (the fixed sequence, every kernel in every step) with HIP events around each
+    force launch on the context's stream."""
     from pis_amd import Engine
 
     eng = Engine(spec, precision)
     eng.load()
     eng.compute_potential()
     _, _, f0 = eng.get_state(0)
-    eng.set_graph_mode(graph)
     if warmup:
         eng.run_nve(spec.dt, warmup, record=True)
     r0 = eng.stats()["rebuilds"]
@@ -155,7 +157,6 @@ def run_drift(spec, precision, warm, steps):
     with Engine(spec, precision) as eng:
         eng.load()
         eng.compute_potential()
-        eng.set_graph_mode(True)
         eng.run_nve(spec.dt, warm, record=False)
         r0 = eng.stats()["rebuilds"]
         t0 = time.perf_counter()
@@ -164,7 +165,7 @@ def run_drift(spec, precision, warm, steps):
         rebuilds = eng.stats()["rebuilds"] - r0
     out = drift_stats(h, spec.n)
     out["warmup"] = warm
-    # the same recorded, graph-replayed steps as the headline, over the whole span
+    # the same recorded steps as the headline, over the whole span
     out["ms_per_step"] = round(1e3 * sec / steps, 5)
     out["atom_steps_per_s"] = round(spec.n * steps / sec, 1)
     out["rebuilds"] = rebuilds
@@ -184,7 +185,6 @@ def run_c3(spec, steps, warm):
             eng.load()
             eng.compute_potential()
             _, _, forces[prec] = eng.get_state(0)
-            eng.set_graph_mode(True)
             eng.run_nve(spec.dt, warm, record=True)
             r0 = eng.stats()["rebuilds"]
             t0 = time.perf_counter()
@@ -206,7 +206,6 @@ def run_c1(steps):
     with Engine(spec, "fp64") as eng:
         eng.load()
         eng.compute_potential()
-        eng.set_graph_mode(True)
         eng.run_nve(spec.dt, 20, record=True)
         t0 = time.perf_counter()
         th = eng.run_nve(spec.dt, steps, record=True)[:, 0, :]
@@ -237,7 +236,7 @@ def run_per_call(spec, steps):
 
 
 def run_thermostats(spec, nvt_steps, npt_steps):
-    """NVT (Nose-Hoover chain, graph replay) and NPT (MTK barostat around the NVT step; the
+    """NVT (Nose-Hoover chain) and NPT (MTK barostat around the NVT step; the
     box becomes general, and the list is kept while the deformation-aware displacement
     check allows) on the same system, mixed precision.  NPT's target is the starting
     pressure with a heavy barostat (tau_p = 50), so the box stays inside its cell grid."""
@@ -311,11 +310,12 @@ def run_dump(spec, steps, cadence):
     return out
 
 
-def run_ensemble(steps, warmup, direct_steps, accuracy=False, tune=True):
+def run_ensemble(steps, warmup, direct_steps, accuracy=False, tune=True, graph=True):
     """Batched ensemble: 512 Kob-Andersen systems (256-32,768 atoms, log-uniform from seed 7,
     density 1.2, T* 0.5-1.5) in one context, mixed precision.  Each step is one replay of
-    the captured step graph (one launch per kernel per LDS staging class over all systems);
-    the same batch with direct launches is timed beside it.  With `tune`, the tiles are the
+    the captured step graph (one launch per kernel per LDS staging class over all systems;
+    `graph` False launches them directly); the same batch with direct launches is timed
+    beside it.  With `tune`, the tiles are the
     autotuner's: every launch class with at least 5 % of the atoms is timed as one batch at
     the candidate tiles around the planner's pick, and moves to another tile only if that
     is 10 % faster (untimed set-up, reported beside)."""
@@ -327,7 +327,8 @@ def run_ensemble(steps, warmup, direct_steps, accuracy=False, tune=True):
     natoms = sum(s.n for s in specs)
     dts = [s.dt for s in specs]
     out = {"n_systems": len(specs), "total_atoms": natoms, "steps": steps,
-           "min_atoms": min(s.n for s in specs), "max_atoms": max(s.n for s in specs)}
+           "min_atoms": min(s.n for s in specs), "max_atoms": max(s.n for s in specs),
+           "stepping": "graph replay" if graph else "direct launches"}
     if tune:
         # the autotuner (pis_amd.tune) in a child process, on the same seeded ensemble
         t0 = time.perf_counter()
@@ -354,7 +355,7 @@ def run_ensemble(steps, warmup, direct_steps, accuracy=False, tune=True):
     with Engine(specs, "mixed") as eng:
         eng.load()
         eng.compute_potential()
-        eng.set_graph_mode(True)
+        eng.set_graph_mode(graph)
         eng.run_nve(dts, warmup, record=False)
         t0 = time.perf_counter()
         eng.run_nve(dts, steps, record=False)
@@ -602,7 +603,9 @@ def main():
     ap.add_argument("--steps", type=int, default=10000)
     ap.add_argument("--warmup", type=int, default=300)
     ap.add_argument("--config", default="c2")
-    ap.add_argument("--no-graph", action="store_true", help="direct launches instead of step-graph replay")
+    ap.add_argument("--no-graph", action="store_true", 
+                    help="the ensemble's steps launched directly instead of replayed from their graph "
+                         "(a lone system's steps are launched by the host either way)")
     ap.add_argument("--cpu-steps", type=int, default=3)
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline and oracle force checks")
     ap.add_argument("--no-fp64", action="store_true", help="skip the FP64 comparison run")
@@ -639,14 +642,14 @@ def main():
     nbar = list_mean(spec)
     log(f"{args.config}: N={spec.n}, mean list length {nbar:.1f}")
 
-    log(f"mixed precision: warmup {args.warmup}, timed {args.steps} steps, graph replay {graph}")
-    mixed = run_gpu(spec, "mixed", args.steps, args.warmup, graph)
+    log(f"mixed precision: warmup {args.warmup}, timed {args.steps} steps, {STEPPING}")
+    mixed = run_gpu(spec, "mixed", args.steps, args.warmup)
     log(f"mixed: {mixed['rate']:.4e} atom-steps/s, {mixed['ms_per_step']:.4f} ms/step, "
         f"force kernel {mixed['force_ms']:.4f} ms, rebuilds {mixed['rebuilds']}")
     fp64 = None
     if not args.no_fp64:
         log(f"fp64: warmup {args.warmup}, timed {args.steps} steps")
-        fp64 = run_gpu(spec, "fp64", args.steps, args.warmup, graph)
+        fp64 = run_gpu(spec, "fp64", args.steps, args.warmup)
         log(f"fp64: {fp64['rate']:.4e} atom-steps/s, {fp64['ms_per_step']:.4f} ms/step, "
             f"force kernel {fp64['force_ms']:.4f} ms, rebuilds {fp64['rebuilds']}")
 
@@ -694,9 +697,10 @@ def main():
 
     ensemble = None
     if args.ensemble_steps:
-        log(f"batched ensemble: 512 KA systems, {args.ensemble_steps} steps, graph replay")
+        log(f"batched ensemble: 512 KA systems, {args.ensemble_steps} steps, "
+            f"{'graph replay' if graph else 'direct launches'}")
         ensemble = run_ensemble(args.ensemble_steps, 100, min(args.ensemble_steps, 1000), accuracy=not args.no_cpu,
-                                tune=not args.no_ensemble_tune)
+                                tune=not args.no_ensemble_tune, graph=graph)
         log(f"ensemble: {ensemble['total_atoms']} atoms, {ensemble['value']:.4e} atom-steps/s "
             f"(direct launches {ensemble.get('direct_launch_value', 0):.4e})")
 
@@ -812,7 +816,7 @@ def main():
             "n_atoms": spec.n,
             "mean_list_length": round(nbar, 2),
             "precision": "mixed",
-            "graph_replay": graph,
+            "stepping": STEPPING,
         },
         "fp64_value": round(fp64["rate"], 1) if fp64 else None,
         "fp64_ms_per_step": round(fp64["ms_per_step"], 5) if fp64 else None,

@@ -3,8 +3,7 @@
 The planner picks each system's tile (cells per workgroup) from a model: lane use of the
 256-thread workgroup times the workgroups per CU that the staging class's LDS allows.
 This module measures instead: it plans the candidate tiles around the model's pick,
-keeps one per distinct (tile, staging class) plan, times a short graph-replayed run of
-each through pis_set_tile_override, and returns the fastest.  The override is process-
+keeps one per distinct (tile, staging class) plan, times a short run of each through pis_set_tile_override, and returns the fastest.  The override is process-
 wide and applies to contexts created afterwards; `apply=True` leaves the winner set.
 
 A batch of systems is tuned per launch class (the systems whose tiles share a staging
@@ -59,14 +58,13 @@ def candidates(spec: SystemSpec, precision: str = "mixed", radius: int = 1, limi
 
 
 def time_tile(spec: SystemSpec, tile, precision: str = "mixed", steps: int = 100, warmup: int = 20) -> float:
-    """Seconds per NVE step of `spec` planned with `tile` (graph replay, no thermo)."""
+    """Seconds per NVE step of `spec` planned with `tile`, alone as it will run (no thermo)."""
     spec = dataclasses.replace(spec, tile=None)
     set_tile_override(tile)
     try:
         with Engine(spec, precision) as eng:
             eng.load()
             eng.compute_potential()
-            eng.set_graph_mode(True)
             eng.run_nve(spec.dt, warmup, record=False)
             t0 = time.perf_counter()
             eng.run_nve(spec.dt, steps, record=False)
@@ -118,9 +116,9 @@ def autotune_ensemble(specs, precision: str = "mixed", steps: int = 60, warmup: 
     pick for its largest system (a tile at which some system of the class would stage more
     atoms than LDS holds is left out), and takes the fastest if it beats the model's pick by
     more than `min_gain`.  A class's gain alone need not carry over to the whole batch,
-    whose classes share the device: on the 512-system Kob-Andersen ensemble one class 9 %
-    faster alone left the replayed step unchanged and made directly launched steps 15 %
-    slower, hence the 10 % default.  Returns (tiles, report): one tile per
+    whose classes share the device: on the 512-system Kob-Andersen ensemble one class 9 to 10 %
+    faster alone leaves the whole batch's step unchanged (1.469 against 1.466 ms replayed, 1.454
+    against 1.453 launched directly), hence the 10 % default.  Returns (tiles, report): one tile per
     system (None keeps the model's pick) and, per class timed, the milliseconds per step
     of every candidate."""
     classes = ensemble_classes(specs, precision)
@@ -162,10 +160,8 @@ __all__ = ["autotune_tiles", "autotune_ensemble", "candidates", "ensemble_classe
 def main(argv=None) -> int:
     """`python -m pis_amd.tune --ka-ensemble N --seed S --nmin A --nmax B [--precision P]`:
     tunes that Kob-Andersen ensemble (workloads.ka_ensemble) and prints one JSON line,
-    {"tiles": [...], "classes": [...], "seconds": t}.  A separate process leaves the
-    caller's device runtime as it was: in one process, directly launched steps of a batch
-    created after the tuner's many short-lived contexts ran 15 % slower (replayed steps
-    did not change)."""
+    {"tiles": [...], "classes": [...], "seconds": t}.  A separate process keeps the tuner's many
+    short-lived contexts and its process-wide override out of the caller's."""
     import argparse
     import json
 
