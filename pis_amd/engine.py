@@ -326,6 +326,7 @@ class LJGpuManager:
         self.precision = precision
         self._engine = None
         self._key = None
+        self._state = None  # positions, velocities, forces as they come back from the device
 
     def insert(self, key, potential: LennardJones):
         self.table[(int(key[0]), int(key[1]))] = potential
@@ -351,20 +352,27 @@ class LJGpuManager:
         if self._engine is None or self._key != key:
             self._engine = Engine(self._spec(atoms), self.precision)
             self._key = key
+            # kept with the engine: arrays made for each call come as fresh pages in a process
+            # whose heap gives them back (1,048,576 atoms, a step 14.5 instead of 11.9 ms)
+            self._state = np.empty((3, atoms.n_atoms, 3))
         return self._engine
 
     def compute_potential(self, atoms: Atoms) -> float:
         eng = self._engine_for(atoms)
         eng.set_state(0, atoms.positions, atoms.velocities, None)
         pe = float(eng.compute_potential()[0])
-        atoms.forces += eng.get_forces(0)
+        force = self._state[2]
+        check(lib().pis_sys_get_state(eng._ptr, 0, None, None, _dptr(force)))
+        atoms.forces += force
         return pe
 
     def verlet_step_nve(self, atoms: Atoms, dt: float) -> float:
         eng = self._engine_for(atoms)
         eng.set_state(0, atoms.positions, atoms.velocities, atoms.forces)
         th = eng.run_nve(dt, 1)
-        atoms.positions[:], atoms.velocities[:], atoms.forces[:] = eng.get_state(0)
+        pos, vel, force = self._state
+        check(lib().pis_sys_get_state(eng._ptr, 0, _dptr(pos), _dptr(vel), _dptr(force)))
+        atoms.positions[:], atoms.velocities[:], atoms.forces[:] = pos, vel, force
         return float(th[0, 0, 0])
 
 

@@ -7,11 +7,13 @@
 * a barostatted run whose grid is planned again on the way: every step has its record;
 * states just below and just above what the pinned staging holds, and records beyond it.
 """
+import tracemalloc
+
 import numpy as np
 import pytest
 
 from oracle import pyoracle as po
-from pis_amd import Engine, plan, workloads as W
+from pis_amd import Atoms, Engine, LennardJones, LJGpuManager, plan, workloads as W
 from tests.test_gpu_npt import sheared
 
 pytestmark = pytest.mark.gpu
@@ -138,6 +140,37 @@ def test_states_around_the_pinned_staging_come_back_whole(n):
         eng.set_state(0, spec.positions)  # no velocities, no forces: zero
         p, v, f = eng.get_state(0)
         assert np.array_equal(p, spec.positions) and not v.any() and not f.any()
+
+
+@pytest.mark.parametrize("n", [4000, PINNED // 72 + 1, 262144])
+def test_per_call_steps_and_forces_make_no_arrays(n):
+    """The drop-in calls bring the state back through arrays that the manager keeps: made anew
+    for each call they are fresh pages, or not, by what the process's heap happens to keep."""
+    spec = W.lj_box(n, 0.8442, 1.0, seed=92)
+    mgr = LJGpuManager(skin=spec.skin, kb=spec.kb, precision="mixed")
+    for ti, tj, eps, sig, rc in spec.pairs:
+        mgr.insert((ti, tj), LennardJones(eps, sig, rc, True))
+    atoms = Atoms(spec.type_ids, spec.masses, spec.positions, spec.velocities, spec.box)
+    mgr.compute_potential(atoms)
+    mgr.verlet_step_nve(atoms, spec.dt)
+    tracemalloc.start()
+    try:
+        for call in (lambda: mgr.verlet_step_nve(atoms, spec.dt), lambda: mgr.compute_potential(atoms)):
+            tracemalloc.reset_peak()
+            base = tracemalloc.get_traced_memory()[0]
+            call()
+            peak = tracemalloc.get_traced_memory()[1] - base
+            print(f"N={n}: {peak} bytes at most", flush=True)
+            assert peak < 24 * n  # less than one array of the state (the engine's key takes 4 n)
+    finally:
+        tracemalloc.stop()
+    # and the arrays are the atoms' own: another set of atoms does not see them
+    other = Atoms(spec.type_ids, spec.masses, spec.positions, spec.velocities, spec.box)
+    kept = atoms.positions.copy(), atoms.velocities.copy(), atoms.forces.copy()
+    mgr.compute_potential(other)
+    mgr.verlet_step_nve(other, spec.dt)
+    for a, b in zip(kept, (atoms.positions, atoms.velocities, atoms.forces)):
+        assert np.array_equal(a, b)
 
 
 def test_records_beyond_the_pinned_staging_equal_those_within_it():
