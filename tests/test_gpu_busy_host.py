@@ -4,6 +4,7 @@ one call and in short ones, and the device does not wait for the thread at every
 import os
 import subprocess
 import sys
+import threading
 import time
 
 import numpy as np
@@ -83,6 +84,30 @@ def test_a_late_thread_changes_no_bit(ens, calls, precision):
     print(f"{precision} {ens}: {a[-1]} rebuilds, {quiet * 1e3:.1f} ms, busy {busy * 1e3:.1f} ms", flush=True)
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+def test_more_runs_than_cpus_change_no_bit():
+    """One engine per thread, more of them than CPUs, several calls each."""
+    spec = W.lj_liquid(8, 0.8442, 1.2, seed=97, skin=0.15)
+    calls = [150, 40, 150]
+    count = min(len(os.sched_getaffinity(0)) + 4, 24)
+    _, alone = run(spec, "mixed", "nve", calls, False)
+    out = [None] * count
+    start = threading.Barrier(count)
+
+    def work(k):
+        start.wait()
+        out[k] = run(spec, "mixed", "nve", calls, False)[1]
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(count)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    print(f"{count} runs", flush=True)
+    for got in out:
+        for x, y in zip(alone, got):
+            assert np.array_equal(x, y)
 
 
 def test_a_late_thread_does_not_stop_the_device():
