@@ -139,8 +139,8 @@ struct SysDev {
     double* scat_x;        // [n] scatter slot -> x (sort key)
     uint4* nbr;            // [(maxnb/8) * npad]
     uint16_t* nnb;         // [npad]
-    double* partial;       // [4 parts][ntile][4]: pe, ke, virial_abs, virial_pair (one part: the first),
-                           // then the number of parts the last force launch wrote
+    double* partial;       // the number of parts the last force launch wrote, 3 unused, then
+                           // [parts][ntile][4]: pe, ke, virial_abs, virial_pair (one part: the first)
     ThermoDev* thermo;     // [thermo_cap]
     const PairParam* pp;   // [ntypes*ntypes]
     const double* mass;    // [ntypes]

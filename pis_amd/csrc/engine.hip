@@ -424,7 +424,9 @@ Layout pis::layout_of(const Plan& p)
     L.sx = take(np * 8);
     L.nbr = take((size_t)(p.maxnb / 8) * np * 16);
     L.nnb = take(np * 2);
-    L.part = take(((size_t)p.ntile * 16 + 1) * 8);
+    // a system of more tiles than four-lane launches take is never launched in parts: room for one
+    // keeps the largest system that fits a given memory as it was
+    L.part = take((4 + (size_t)p.ntile * 4 * class_lanes(p.ntile)) * 8);
     L.pp = take(p.pp.size() * sizeof(PairParam));
     L.m = take(p.mass.size() * 8);
     L.nhc = take(NHC_COUNT * 8);

@@ -2197,7 +2197,7 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
             sum[3] += acc.wp;
         }
     }
-    double* P = s.partial + 4 * ((size_t)part * s.ntile + w.idx);
+    double* P = s.partial + 4 * (1 + (size_t)part * s.ntile + w.idx);
     if constexpr (KL == 1) {
         block_sum4(sum, lds.rtmp);
     } else {
@@ -2215,7 +2215,7 @@ __global__ __launch_bounds__(kTileThreads, (ForceWaves<MIXED, KIND, KL>::value))
             sum[k] = (lds.rtmp[k] + lds.rtmp[4 + k]) + (lds.rtmp[8 + k] + lds.rtmp[12 + k]);
     }
     if (threadIdx.x == 0) {
-        if (w.idx == 0 && part == 0) s.partial[16 * (size_t)s.ntile] = KL;
+        if (w.idx == 0 && part == 0) s.partial[0] = KL;
         P[0] = sum[0];
         P[1] = sum[1];
         P[2] = sum[2];
@@ -2253,10 +2253,10 @@ __device__ double nhc_kinetic(const double* c)
 __device__ __forceinline__ void sum_partials(const SysDev& s, double* v, double* rtmp)
 {
     v[0] = v[1] = v[2] = v[3] = 0.0;
-    const __attribute__((address_space(1))) double* P = gbl(static_cast<const double*>(s.partial));
+    const __attribute__((address_space(1))) double* P = gbl(static_cast<const double*>(s.partial)) + 4;
     const int bd = blockDim.x;
     int t = threadIdx.x;
-    if (P[16 * s.ntile] > 1.0) {  // parts of the launch that wrote them
+    if (P[-4] > 1.0) {  // parts of the launch that wrote them
         // four parts per tile, added as block_sum4 adds a tile's four waves
         for (; t < s.ntile; t += bd)
 #pragma unroll
