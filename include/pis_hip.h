@@ -122,7 +122,7 @@ typedef struct pis_plan_info {
 typedef struct pis_stats {
     uint64_t steps;
     uint64_t rebuilds;
-    uint64_t force_launches;
+    uint64_t force_launches; /* of steps and force calls; one per step or call, over all classes */
     double force_kernel_ms; /* summed HIP-event time of force launches while timing is on */
     uint64_t timed_force_launches;
     int32_t neighbor_capacity;

@@ -277,6 +277,8 @@ class Engine:
         return {f[0]: getattr(s, f[0]) for f in _capi.Stats._fields_}
 
     def set_graph_mode(self, enable: bool):
+        """Replay a captured graph per step of a batch instead of launching each kernel.  A lone
+        system's steps are launched by the host either way, list rebuilds only when due."""
         check(lib().pis_set_graph_mode(self._ptr, 1 if enable else 0))
 
     def set_kernel_timing(self, enable: bool):
