@@ -1962,18 +1962,26 @@ pis_status pis_get_list_digest(pis_ctx* ctx, uint32_t* counts, uint64_t* hashes)
     PIS_HIP(hipStreamSynchronize(ctx->stream));
     PIS_TRY(check_flags(ctx));
     const size_t n = (size_t)ctx->sys[0].plan.n;
-    void* d_out = nullptr;
-    PIS_HIP(hipMalloc(&d_out, n * 12));
-    uint64_t* d_hash = (uint64_t*)d_out;
+    // a state's transfer has left more than this in d_xfer; the way back is that of a state's arrays
+    PIS_TRY(ensure_xfer(ctx, n * 12));
+    uint64_t* d_hash = (uint64_t*)ctx->d_xfer;
     uint32_t* d_cnt = (uint32_t*)(d_hash + n);
+    const bool pinned = n * 12 <= kPinnedMax;
+    if (pinned) PIS_TRY(ensure_pin(ctx, n * 12));
     for (const auto& k : ctx->classes)
         launch_list_digest(ctx->stream, ctx->d_sys, ctx->d_tile_work + k.first, k.count, k.scap, d_cnt, d_hash);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(hashes, d_hash, n * 8, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(counts, d_cnt, n * 4, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(d_out);
-    if (e != hipSuccess) return fail(PIS_ERR_HIP, std::string("list digest: ") + hipGetErrorString(e));
+    PIS_HIP(hipGetLastError());
+    if (pinned) {
+        PIS_HIP(hipMemcpyAsync(ctx->h_pin, d_hash, n * 12, hipMemcpyDeviceToHost, ctx->stream));
+    } else {
+        PIS_HIP(hipMemcpyAsync(hashes, d_hash, n * 8, hipMemcpyDeviceToHost, ctx->stream));
+        PIS_HIP(hipMemcpyAsync(counts, d_cnt, n * 4, hipMemcpyDeviceToHost, ctx->stream));
+    }
+    PIS_HIP(hipStreamSynchronize(ctx->stream));
+    if (pinned) {
+        memcpy(hashes, ctx->h_pin, n * 8);
+        memcpy(counts, (char*)ctx->h_pin + n * 8, n * 4);
+    }
     return PIS_OK;
 }
 

@@ -142,6 +142,26 @@ def test_states_around_the_pinned_staging_come_back_whole(n):
         assert np.array_equal(p, spec.positions) and not v.any() and not f.any()
 
 
+# 12 bytes per atom come back
+@pytest.mark.parametrize("n", [2, 4000, PINNED // 12, PINNED // 12 + 1])
+def test_list_digests_around_the_pinned_staging_match_the_list(n):
+    spec = W.lj_box(n, 0.3 if n > 2 else 0.002, 1.0, seed=93)
+    with Engine(spec, "mixed") as eng:
+        eng.load()
+        counts, hashes = eng.list_digest()
+        offsets, idx = eng.neighbor_list()
+        again = eng.list_digest()
+    assert np.array_equal(counts, np.diff(offsets))
+    with np.errstate(over="ignore"):  # splitmix64's output function, summed over each row
+        x = idx.astype(np.uint64) + np.uint64(0x9E3779B97F4A7C15)
+        x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        x = (x ^ (x >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        x ^= x >> np.uint64(31)
+        total = np.concatenate([np.zeros(1, dtype=np.uint64), np.cumsum(x, dtype=np.uint64)])
+        assert np.array_equal(hashes, total[offsets[1:]] - total[offsets[:-1]])
+    assert np.array_equal(again[0], counts) and np.array_equal(again[1], hashes)
+
+
 @pytest.mark.parametrize("n", [4000, PINNED // 72 + 1, 262144])
 def test_per_call_steps_and_forces_make_no_arrays(n):
     """The drop-in calls bring the state back through arrays that the manager keeps: made anew
